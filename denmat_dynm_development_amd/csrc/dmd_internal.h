@@ -37,6 +37,10 @@ inline unsigned nblk(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); 
 #define DMD_TILE4_R 32
 #define DMD_TILE4_GROUP 1
 #define DMD_TILE4_CMAX 2048
+// what a workgroup's prologue and flush cost, in pairs of its stream (the
+// chunk planner's weights; from sweeps of the chunk length)
+#define DMD_TILE_OVER 100
+#define DMD_TILE4_OVER 16
 
 // nb = 4 blocked pair record (512 complex elements, P1 then P2): offset of
 // P_mat[row][col] for U elements per 16-byte unit.  Lane l = 4 (row/4) +

@@ -29,6 +29,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <functional>
 #include <memory>
 #include <string>
 #include <vector>
@@ -894,6 +895,66 @@ int set_clock(dmd_scatt *h, double t0, double dt, long long step)
 
 }  // namespace dmd
 
+namespace dmd {
+// Pairs per workgroup of the tile kernels: the length L a tile is cut at,
+// into ceil(size / L) pieces of equal length (a multiple of `unit`).  One
+// workgroup per CU already streams at the HBM rate, so what a length costs is
+// the CU that is handed the most: the pieces are dealt in order to the least
+// loaded of the 256 CUs, a piece counting its pairs plus `over` pairs for its
+// prologue and flush, and the length with the smallest largest load is taken.
+// `tail` adds that many longest pieces: the nb = 4 kernels need their two or
+// three workgroups per CU to keep the rate, so a last piece left alone on its
+// CU runs slowly.  Against the fixed lengths before (max(512, pairs / 4096) and
+// 2048), contraction and assembly: nb = 2, 0.96 M pairs 95 -> 82 us, 0.44 M
+// 47.5 -> 42 us; nb = 4 FP64, 0.59 M pairs 1050 -> 765-825 us (6.3 TB/s),
+// 23 k pairs 485 -> 44 us; BF16, 1.6 M pairs 1046 -> 800 us; 15.5 M pairs
+// (nb = 2) unchanged.
+static int64_t plan_chunk_len(const std::vector<int64_t> &sizes, int64_t unit, int64_t over, double tail,
+                              int64_t lo, int64_t hi)
+{
+    constexpr int kCu = 256;
+    int64_t at_lo = 0, best = hi, seen_pieces = 0, seen_longest = 0;
+    for (int64_t n : sizes) at_lo += (n + lo - 1) / lo;
+    if (at_lo <= kCu) return lo;  // a CU for every shortest piece
+    double best_cost = 1e300;
+    std::vector<int64_t> cu;
+    for (int64_t L = hi; L >= lo; L = std::min(L - unit, L * 15 / 16 / unit * unit)) {
+        int64_t pieces = 0, load = 0, longest = 0;
+        for (int64_t n : sizes) {
+            if (!n) continue;
+            const int64_t m = (n + L - 1) / L, len = ((n + m - 1) / m + unit - 1) / unit * unit, k = (n + len - 1) / len;
+            pieces += k;
+            load += k * (len + over);
+            longest = std::max(longest, len + over);
+        }
+        if (pieces == seen_pieces && longest == seen_longest) continue;  // the same pieces as the last length
+        seen_pieces = pieces;
+        seen_longest = longest;
+        // the mean load is the least the largest can be; with many pieces it is
+        // the estimate, with half a piece at the end
+        double cost = std::max((double)load / kCu, (double)longest) + tail * (double)longest;
+        if (pieces > 16 * kCu) {
+            cost = (double)load / kCu + (0.5 + tail) * (double)longest;
+        } else if (cost < best_cost) {
+            cu.assign(kCu, 0);  // a heap by load, least first
+            const auto more = std::greater<int64_t>();
+            for (int64_t n : sizes) {
+                if (!n) continue;
+                const int64_t m = (n + L - 1) / L, len = ((n + m - 1) / m + unit - 1) / unit * unit;
+                for (int64_t a = 0; a < n; a += len) {
+                    std::pop_heap(cu.begin(), cu.end(), more);
+                    cu.back() += len + over;
+                    std::push_heap(cu.begin(), cu.end(), more);
+                }
+            }
+            cost = (double)*std::max_element(cu.begin(), cu.end()) + tail * (double)longest;
+        }
+        if (cost < best_cost) { best_cost = cost; best = L; }
+    }
+    return best;
+}
+}  // namespace dmd
+
 extern "C" const char *dmd_scatt_last_error(void) { return g_err.c_str(); }
 extern "C" int dmd_scatt_version(void) { return 1; }
 
@@ -952,13 +1013,13 @@ extern "C" int dmd_scatt_create(int64_t nk, int nb, int64_t n_pairs, const uint6
     const bool lane_perm = nb <= 2;  // nb = 4: a chunk is walked by quarters, no slot permutation
     h->tile_R = R;
     // Slots: physical positions of P.  With tiles, each tile's pairs (in
-    // (k, k') order) are cut into chunks of at most cmax pairs; a chunk of n
-    // pairs occupies m = ceil(n/64) blocks of 64 slots, pair L of the chunk
-    // going to slot (L % m) * 64 + L / m.  So lane l of a wavefront walking
-    // the chunk block by block meets pairs l*m, l*m+1, ... (one k for long
-    // runs; the 64 lanes sit on different rows), while each block of 64 slots
-    // is still read as 8 coalesced SoA granules.  Unused slots hold P = 0 and
-    // are never read.
+    // (k, k') order) are cut into chunks of equal length (plan_chunk_len); a
+    // chunk of n pairs occupies m = ceil(n/64) blocks of 64 slots, pair L of
+    // the chunk going to slot (L % m) * 64 + L / m.  So lane l of a wavefront
+    // walking the chunk block by block meets pairs l*m, l*m+1, ... (one k for
+    // long runs; the 64 lanes sit on different rows), while each block of 64
+    // slots is still read as 8 coalesced SoA granules.  Unused slots hold P =
+    // 0 and are never read.
     std::vector<int64_t> phys;  // slot -> file index, -1 for padding
     std::vector<int64_t> cbeg;
     std::vector<int32_t> clen;
@@ -966,8 +1027,6 @@ extern "C" int dmd_scatt_create(int64_t nk, int nb, int64_t n_pairs, const uint6
     int64_t nslots = n_pairs;
     if (R) {
         const int64_t nbk = (nk + R - 1) / R;
-        const int64_t cmax = lane_perm ? std::min<int64_t>(16384, std::max<int64_t>(512, n_pairs / 4096)) / 64 * 64
-                                       : DMD_TILE4_CMAX;
         const int64_t pad = lane_perm ? 64 : 4;
         // nb <= 2: tiles (K/R, K'/R); nb = 4: row panels K/R (all k' of the rows)
         const int64_t nbc = lane_perm ? nbk : 1, ntile = nbk * nbc;
@@ -985,10 +1044,20 @@ extern "C" int dmd_scatt_create(int64_t nk, int nb, int64_t n_pairs, const uint6
                 byt[cur[tile_of(f)]++] = f;
             }
         }
+        // a wavefront takes 64 slots (nb <= 2) or a workgroup 16 pairs (nb = 4) at a time
+        const int64_t unit = lane_perm ? 64 : 16;
+        std::vector<int64_t> sizes(ntile);
+        for (int64_t t = 0; t < ntile; t++) sizes[t] = tc[t + 1] - tc[t];
+        const int64_t cut = lane_perm ? plan_chunk_len(sizes, unit, DMD_TILE_OVER, 0.0, 256, 16384)
+                                      : plan_chunk_len(sizes, unit, DMD_TILE4_OVER, 1.0, 64, DMD_TILE4_CMAX);
+        auto len_of = [&](int64_t t) {  // piece length of tile t
+            const int64_t m = (sizes[t] + cut - 1) / cut;
+            return m ? ((sizes[t] + m - 1) / m + unit - 1) / unit * unit : unit;
+        };
         nslots = 0;
         for (int64_t t = 0; t < ntile; t++)
-            for (int64_t a = tc[t]; a < tc[t + 1]; a += cmax) {
-                int64_t n = std::min<int64_t>(cmax, tc[t + 1] - a);
+            for (int64_t a = tc[t], len = len_of(t); a < tc[t + 1]; a += len) {
+                int64_t n = std::min<int64_t>(len, tc[t + 1] - a);
                 cbeg.push_back(nslots);
                 clen.push_back((int32_t)n);
                 cij.push_back(make_int2((int)(t / nbc), (int)(t % nbc)));
@@ -997,7 +1066,7 @@ extern "C" int dmd_scatt_create(int64_t nk, int nb, int64_t n_pairs, const uint6
         phys.assign(nslots, -1);
         int64_t c = 0;
         for (int64_t t = 0; t < ntile; t++)
-            for (int64_t a = tc[t]; a < tc[t + 1]; a += cmax, c++) {
+            for (int64_t a = tc[t], len = len_of(t); a < tc[t + 1]; a += len, c++) {
                 const int64_t n = clen[c], m = (n + 63) / 64;
                 for (int64_t L = 0; L < n; L++)
                     phys[cbeg[c] + (lane_perm ? (L % m) * 64 + L / m : L)] = byt[a + L];
