@@ -21,7 +21,9 @@
 // nk_full, doubled with exchange.  The density matrices are Hermitian and
 // read from their upper triangle, as the reference's zhemm does.
 //
-// MI355X mapping: nb <= 2, one wavefront per stored pair (k_ee_pair2): the
+// MI355X mapping: nb <= 2 in the Lindblad form without exchange, the pairs
+// grouped by q (k_ee_group below); the other nb <= 2 forms, and pairs too
+// scattered over q, one wavefront per stored pair (k_ee_pair2): the
 // lanes test 64 k3 at a time against the energy window and queue the
 // survivors in LDS, so every term runs with all lanes busy, and one term forms
 // the overlaps and A2 blocks once for P1 and P2; nb > 2, one thread per P
@@ -518,6 +520,437 @@ __global__ __launch_bounds__(256) void k_ee_pair2(int64_t n, const uint64_t *__r
     }
 }
 
+// ---------------------------------------------------------------------------
+// nb <= 2 without exchange in the Lindblad form: pairs grouped by q = k1 - k2.
+//
+// There A2(pq)_xy = o12_pq o34_xy G_pq(xy) with o12 the pair's v <k1 p|k2 q>,
+// o34 = <k3 x|k4 y>, G the real Gaussian of e1p - e2q + e34_xy, and A1 = A2, so
+//   P[.., ..] = o12_pq conj(o12_p'q') S[pq, p'q'],
+//   S = sum_k3 G W G^T,  W[(x'y'), (xy)] = D o34_x'y' conj(o34_xy),
+// D the product of the two density matrices (L[x x'] R[y' y]; the linearize_dPee
+// form fl[x] R'[y' y] at x = x' plus L'[x x'] fr[y] at y = y').  W is Hermitian
+// and depends on (k3, q) only: k_ee_qtab forms k4, e34 and the two forms' W once
+// per (q, k3), and every pair of that q only pays the Gaussians and the two
+// real-by-Hermitian products (16 exponentials and about 350 FMAs per k3 at
+// nb = 2, against about 1700 with the overlaps and the products of density
+// matrices per pair).  k_ee_pair2 spent its time on latency besides: 452
+// registers (one wave per SIMD), k4's integer divisions and some thirty
+// dependent gathers per k3.  Rebuild of 100 k pairs on a 12^3 mesh: 20.7 ms
+// -> 3.9 ms in k_ee_group (FP64 issue slots 62 % full) and 0.7 ms in k_ee_qtab.
+//
+// Layout: tab[q row][tile of kEeTile k3][field][k3], fields e34 | W of P1 | W of
+// P2 (NP real diagonals, then re and im of the upper elements).  A workgroup
+// stages a tile (36 doubles x 512 k3 = 144 KiB of LDS, so one workgroup of
+// eight waves per CU) for up to eight pairs of one q, a wavefront each; a
+// group of fewer pairs gives every pair two, four or eight wavefronts that
+// share its k3.  The window test queues the tile's k3 of a pair in LDS, so the
+// terms run with all lanes busy.
+// ---------------------------------------------------------------------------
+constexpr int kEeTile = 512;   // k3 per staged tile
+constexpr int kEeGroup = 8;    // pairs (wavefronts) per workgroup
+
+template <int NB>
+struct EeTab {
+    static constexpr int NP = NB * NB, NH = NP * NP, F = NP + 2 * NH;
+};
+// first field of the upper element (a, b), a < b, inside a W
+template <int NP>
+__device__ constexpr int ee_up(int a, int b)
+{
+    return NP + 2 * (a * NP - a * (a + 1) / 2 + (b - a - 1));
+}
+
+template <int NB>
+__global__ __launch_bounds__(256) void k_ee_qtab(int64_t nrow, int64_t ntile, const int *__restrict__ rowcell, EeArgs a,
+                                                 double *__restrict__ tab)
+{
+    using T = EeTab<NB>;
+    constexpr int NB2 = NB * NB, NP = T::NP, NH = T::NH;
+    const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t row = idx / (ntile * kEeTile), c3 = idx - row * (ntile * kEeTile);
+    if (row >= nrow) return;
+    double *t = tab + ((row * ntile + c3 / kEeTile) * T::F) * kEeTile + c3 % kEeTile;
+    int64_t c4 = -1;
+    if (c3 < a.nk) {
+        const int q = rowcell[row], qz = q % a.m2, qy = (q / a.m2) % a.m1, qx = q / (a.m2 * a.m1);
+        int x = a.ik3[3 * c3] + qx, y = a.ik3[3 * c3 + 1] + qy, z = a.ik3[3 * c3 + 2] + qz;
+        x -= x >= a.m0 ? a.m0 : 0;
+        y -= y >= a.m1 ? a.m1 : 0;
+        z -= z >= a.m2 ? a.m2 : 0;
+        const int g = a.grid[(x * a.m1 + y) * a.m2 + z];
+        c4 = g == INT_MAX ? -1 : (int64_t)g;
+    }
+    if (c4 < 0) {  // never inside the window
+#pragma unroll
+        for (int f = 0; f < T::F; f++) t[f * kEeTile] = f < NP ? 1e300 : 0.0;
+        return;
+    }
+    const double *e3 = a.e + c3 * NB, *e4 = a.e + c4 * NB, *f3 = a.f + c3 * NB, *f4 = a.f + c4 * NB;
+    double2 o[NP], oo[NP][NP];
+#pragma unroll
+    for (int x = 0; x < NB; x++)
+#pragma unroll
+        for (int y = 0; y < NB; y++) {
+            o[x * NB + y] = ee_ov<NB>(a, c3, c4, x, y);
+            t[(x * NB + y) * kEeTile] = e3[x] - e4[y];
+        }
+#pragma unroll
+    for (int i = 0; i < NP; i++)
+#pragma unroll
+        for (int j = i; j < NP; j++) oo[i][j] = cmulc(o[i], o[j]);
+#pragma unroll
+    for (int which = 0; which < 2; which++) {
+        const double2 *L = nullptr, *R = nullptr;  // P1: dm1_k3, dm_k4; P2: dm_k3, dm1_k4
+        if (a.dm) {
+            L = (which ? a.dm : a.dm1) + c3 * NB2;
+            R = (which ? a.dm1 : a.dm) + c4 * NB2;
+        }
+        double fl[NB], fr[NB];
+#pragma unroll
+        for (int x = 0; x < NB; x++) {
+            fl[x] = which ? f3[x] : 1 - f3[x];
+            fr[x] = which ? 1 - f4[x] : f4[x];
+        }
+        double *w = t + (NP + which * NH) * kEeTile;
+#pragma unroll
+        for (int i = 0; i < NP; i++)
+#pragma unroll
+            for (int j = i; j < NP; j++) {
+                const int xp = i / NB, yp = i % NB, x = j / NB, y = j % NB;
+                double2 d = make_double2(0.0, 0.0);
+                if (L && a.dP) {
+                    if (x == xp) {
+                        const double2 r = ee_hus<NB>(R, fr, yp, y);
+                        d = make_double2(fl[x] * r.x, fl[x] * r.y);
+                    }
+                    if (y == yp) {
+                        const double2 l = ee_hus<NB>(L, fl, x, xp);
+                        d = make_double2(d.x + l.x * fr[y], d.y + l.y * fr[y]);
+                    }
+                } else if (L) {
+                    d = cmul(ee_hu<NB>(L, x, xp), ee_hu<NB>(R, yp, y));
+                } else if (i == j) {
+                    d = make_double2(fl[x] * fr[y], 0.0);
+                }
+                const double2 v = cmul(d, oo[i][j]);
+                if (i == j) {
+                    w[i * kEeTile] = v.x;
+                } else {
+                    w[ee_up<NP>(i, j) * kEeTile] = v.x;
+                    w[(ee_up<NP>(i, j) + 1) * kEeTile] = v.y;
+                }
+            }
+    }
+}
+
+// N Gaussian factors exp(x[i]), x <= 0, side by side (no branch, so the N
+// chains overlap; two waves per SIMD leave a single chain's latency bare).
+// exp(x) = 2^n e^r with n = rint(x / ln 2) and r = x - n ln 2 from ln 2 in two
+// parts (Cody and Waite), e^r its Taylor series to r^13: |r| < 0.347, so the
+// rest is under 4e-18.  Underflows to 0 through ldexp.
+template <int N>
+__device__ __forceinline__ void ee_exp_n(const double x[N], double g[N])
+{
+    constexpr double kLog2e = 1.4426950408889634074;
+    constexpr double kLn2Hi = 0x1.62e42fefa3800p-1;  // 42 bits: n kLn2Hi is exact
+    constexpr double kLn2Lo = 5.497923018708371155e-14;  // ln 2 - kLn2Hi
+    constexpr double kC[14] = { 1., 1., 1. / 2, 1. / 6, 1. / 24, 1. / 120, 1. / 720, 1. / 5040, 1. / 40320,
+                                1. / 362880, 1. / 3628800, 1. / 39916800, 1. / 479001600, 1. / 6227020800. };
+    double n[N], r[N];
+#pragma unroll
+    for (int i = 0; i < N; i++) n[i] = rint(x[i] * kLog2e);
+#pragma unroll
+    for (int i = 0; i < N; i++) r[i] = fma(-n[i], kLn2Lo, fma(-n[i], kLn2Hi, x[i]));
+#pragma unroll
+    for (int i = 0; i < N; i++) g[i] = kC[13];
+#pragma unroll
+    for (int k = 12; k >= 0; k--)
+#pragma unroll
+        for (int i = 0; i < N; i++) g[i] = fma(g[i], r[i], kC[k]);
+#pragma unroll
+    for (int i = 0; i < N; i++) g[i] = ldexp(g[i], (int)fmax(n[i], -2000.0));
+}
+
+// One k3 of one pair: S += G W G^T of both forms (upper elements).  w: the
+// staged tile at this k3; g: the Gaussians G[pq][xy].
+template <int NB>
+__device__ __forceinline__ void ee_group_term(const double *w, const double g[NB * NB][NB * NB], double *S)
+{
+    using T = EeTab<NB>;
+    constexpr int NP = T::NP, NH = T::NH;
+#pragma unroll
+    for (int which = 0; which < 2; which++) {
+        double W[NH];
+#pragma unroll
+        for (int f = 0; f < NH; f++) W[f] = w[(NP + which * NH + f) * kEeTile];
+        double *s = S + which * NH;
+#pragma unroll
+        for (int p = 0; p < NP; p++) {
+            double tr[NP], ti[NP];  // row p of G W
+#pragma unroll
+            for (int b = 0; b < NP; b++) {
+                tr[b] = g[p][b] * W[b];
+                ti[b] = 0.0;
+#pragma unroll
+                for (int c = 0; c < NP; c++) {
+                    if (c < b) {
+                        tr[b] = fma(g[p][c], W[ee_up<NP>(c, b)], tr[b]);
+                        ti[b] = fma(g[p][c], W[ee_up<NP>(c, b) + 1], ti[b]);
+                    } else if (c > b) {
+                        tr[b] = fma(g[p][c], W[ee_up<NP>(b, c)], tr[b]);
+                        ti[b] = fma(-g[p][c], W[ee_up<NP>(b, c) + 1], ti[b]);
+                    }
+                }
+            }
+#pragma unroll
+            for (int b = 0; b < NP; b++) s[p] = fma(tr[b], g[p][b], s[p]);
+#pragma unroll
+            for (int q = p + 1; q < NP; q++)
+#pragma unroll
+                for (int b = 0; b < NP; b++) {
+                    s[ee_up<NP>(p, q)] = fma(tr[b], g[q][b], s[ee_up<NP>(p, q)]);
+                    s[ee_up<NP>(p, q) + 1] = fma(ti[b], g[q][b], s[ee_up<NP>(p, q) + 1]);
+                }
+        }
+    }
+}
+
+// P1, P2 of the pairs of one group (grp: q row, first entry of order, pairs).
+template <int NB>
+__global__ __launch_bounds__(64 * kEeGroup, 2) void k_ee_group(const int4 *__restrict__ grp, int row0, int64_t ntile,
+                                                               const int *__restrict__ order,
+                                                               const uint64_t *__restrict__ k1,
+                                                               const uint64_t *__restrict__ k2, EeArgs a, EimpConst c,
+                                                               const double *__restrict__ tab,
+                                                               double2 *__restrict__ P1, double2 *__restrict__ P2)
+{
+    using T = EeTab<NB>;
+    constexpr int NB2 = NB * NB, NB4 = NB2 * NB2, NP = T::NP, NH = T::NH, F = T::F;
+    __shared__ double tile[F * kEeTile];
+    __shared__ uint16_t queue[kEeGroup][kEeTile];
+    __shared__ double red[kEeGroup][2 * NH];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int4 G = grp[blockIdx.x];
+    const int cnt = G.z, wpp = cnt > 4 ? 1 : (cnt > 2 ? 2 : (cnt > 1 ? 4 : 8));  // wavefronts per pair
+    const int pi = wv / wpp, sub = wv - pi * wpp;
+    const bool active = pi < cnt;
+    const int64_t fp = order[G.y + (active ? pi : 0)];
+    const int64_t A = (int64_t)k1[fp], B = (int64_t)k2[fp];
+    double d12[NP], dmin = 1e300, dmax = -1e300;
+#pragma unroll
+    for (int p = 0; p < NB; p++)
+#pragma unroll
+        for (int q = 0; q < NB; q++) {
+            d12[p * NB + q] = a.e[A * NB + p] - a.e[B * NB + q];
+            dmin = fmin(dmin, d12[p * NB + q]);
+            dmax = fmax(dmax, d12[p * NB + q]);
+        }
+    double S[2 * NH];
+#pragma unroll
+    for (int i = 0; i < 2 * NH; i++) S[i] = 0.0;
+    const uint64_t below = (1ull << lane) - 1ull;
+    for (int64_t tl = 0; tl < ntile; tl++) {
+        const dmd_dv2 *src = (const dmd_dv2 *)(tab + ((int64_t)(G.x - row0) * ntile + tl) * F * kEeTile);
+        // all of a thread's loads in flight at once (one by one the staging took
+        // longer than the terms), under the other waves' last terms
+        constexpr int kThreads = 64 * kEeGroup, kWords = F * kEeTile / 2, kPer = (kWords + kThreads - 1) / kThreads;
+        dmd_dv2 v[kPer];
+#pragma unroll
+        for (int i = 0; i < kPer; i++) {
+            const int w = i * kThreads + threadIdx.x;
+            v[i] = src[w < kWords ? w : 0];
+        }
+        __syncthreads();  // the previous tile is read
+#pragma unroll
+        for (int i = 0; i < kPer; i++) {
+            const int w = i * kThreads + threadIdx.x;
+            if (w < kWords) ((dmd_dv2 *)tile)[w] = v[i];
+        }
+        __syncthreads();
+        if (!active) continue;
+        int qlen = 0;  // wavefront-uniform
+        for (int blk = sub; blk < kEeTile / 64; blk += wpp) {
+            const int j = blk * 64 + lane;
+            double lo = tile[j], hi = lo;
+#pragma unroll
+            for (int f = 1; f < NP; f++) {
+                lo = fmin(lo, tile[f * kEeTile + j]);
+                hi = fmax(hi, tile[f * kEeTile + j]);
+            }
+            const bool ok = dmin + lo < c.m.ethr && dmax + hi > -c.m.ethr;  // some A2 entry inside the window
+            const uint64_t m = __ballot(ok);
+            if (ok) queue[wv][qlen + __popcll(m & below)] = (uint16_t)j;
+            qlen += __popcll(m);
+        }
+        __builtin_amdgcn_wave_barrier();
+        for (int r = 0; r < qlen; r += 64) {
+            const bool live = r + lane < qlen;
+            const double *w = tile + queue[wv][live ? r + lane : r];
+            double g[NP][NP];
+#pragma unroll
+            for (int x = 0; x < NP; x++) {
+                const double e34 = w[x * kEeTile];
+                double arg[NP], ex[NP];
+                bool in[NP];
+#pragma unroll
+                for (int p = 0; p < NP; p++) {
+                    const double de = d12[p] + e34;
+                    in[p] = live && fabs(de) < c.m.ethr;
+                    arg[p] = c.prefac_exp * (de * de);
+                }
+                ee_exp_n<NP>(arg, ex);
+#pragma unroll
+                for (int p = 0; p < NP; p++) g[p][x] = in[p] ? ex[p] : 0.0;
+            }
+            ee_group_term<NB>(w, g, S);
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+    // the lanes' sums through LDS: a wavefront writes its 2 NH values of 64
+    // lanes and each lane adds a share of one value's (a shuffle tree over 32
+    // values took a tenth of the kernel)
+    __syncthreads();  // the last tile is read
+    constexpr int kPart = NH > 1 ? 2 : 8;  // lanes per value
+    static_assert(kEeGroup * 2 * NH * 66 <= F * kEeTile && 2 * NH * kPart <= 64, "the sums fit the tile");
+    double *mine = tile + wv * (2 * NH * 66);
+#pragma unroll
+    for (int i = 0; i < 2 * NH; i++) mine[i * 66 + lane] = S[i];
+    __builtin_amdgcn_wave_barrier();
+    if (lane < 2 * NH * kPart) {
+        const double *m = mine + (lane / kPart) * 66 + (lane % kPart) * (64 / kPart);
+        double v = 0.0;
+#pragma unroll
+        for (int k = 0; k < 64 / kPart; k++) v += m[k];
+#pragma unroll
+        for (int off = 1; off < kPart; off <<= 1) v += __shfl_xor(v, off, 64);
+        if (lane % kPart == 0) red[wv][lane / kPart] = v;
+    }
+    __syncthreads();
+    if (!active || sub || lane >= 2 * NB4) return;
+    // element (i1 i2),(i3 i4): P1 from (i1 i3), (i2 i4); P2 from (i3 i1), (i4 i2)
+    const int which = lane / NB4, el = lane % NB4;
+    const int i1 = el / (NB * NB2), i2 = (el / NB2) % NB, i3 = (el / NB) % NB, i4 = el % NB;
+    const int p = which ? i3 : i1, q = which ? i1 : i3, r = which ? i4 : i2, s = which ? i2 : i4;
+    const int u = p * NB + q, v = r * NB + s;
+    auto sum = [&](int f) {
+        double x = 0.0;
+        for (int k = 0; k < wpp; k++) x += red[wv + k][which * NH + f];
+        return x;
+    };
+    double2 out = make_double2(0.0, 0.0);
+    if (A != B) {
+        const int lo = u < v ? u : v, hi = u < v ? v : u;
+        const int f = NP + 2 * (lo * NP - lo * (lo + 1) / 2 + (hi - lo - 1));
+        double2 x = u == v ? make_double2(sum(u), 0.0) : make_double2(sum(f), sum(f + 1));
+        if (u > v) x.y = -x.y;
+        const double v12 = a.vq_pair ? a.vq_pair[fp] : ee_v(a, c.m, A, B);
+        double2 o1 = ee_ov<NB>(a, A, B, p, q), o2 = ee_ov<NB>(a, A, B, r, s);
+        o1 = make_double2(o1.x * v12, o1.y * v12);
+        o2 = make_double2(o2.x * v12, o2.y * v12);
+        out = cmul(cmulc(o1, o2), x);
+        out = make_double2(out.x * a.pfac, out.y * a.pfac);
+    }
+    (which ? P2 : P1)[fp * NB4 + el] = out;
+}
+
+// The pairs of a chunk by q: count per mesh cell (a pair's rank in its cell is
+// its order of arrival; every pair is independent), a scan over the cells that
+// numbers the non-empty ones (rows), their pairs and their groups, and the
+// pairs' places.
+__global__ __launch_bounds__(256) void k_ee_qcell(int64_t n, const uint64_t *__restrict__ k1,
+                                                  const uint64_t *__restrict__ k2, EeArgs a, int *__restrict__ cnt,
+                                                  int *__restrict__ cell, int *__restrict__ rank)
+{
+    const int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (f >= n) return;
+    const int64_t A = (int64_t)k1[f], B = (int64_t)k2[f];
+    int x = a.ik3[3 * A] - a.ik3[3 * B], y = a.ik3[3 * A + 1] - a.ik3[3 * B + 1], z = a.ik3[3 * A + 2] - a.ik3[3 * B + 2];
+    x += x < 0 ? a.m0 : 0;
+    y += y < 0 ? a.m1 : 0;
+    z += z < 0 ? a.m2 : 0;
+    const int q = (x * a.m1 + y) * a.m2 + z;
+    cell[f] = q;
+    rank[f] = atomicAdd(cnt + q, 1);
+}
+// Exclusive sums of (rows, pairs, groups) over a block of 256 threads.
+__device__ __forceinline__ int3 ee_scan256(int3 v, int3 *total)
+{
+    __shared__ int3 part[256];
+    const int t = threadIdx.x;
+    int3 x = v;
+    part[t] = x;
+    __syncthreads();
+    for (int o = 1; o < 256; o <<= 1) {
+        int3 y = make_int3(0, 0, 0);
+        if (t >= o) y = part[t - o];
+        __syncthreads();
+        x = make_int3(x.x + y.x, x.y + y.y, x.z + y.z);
+        part[t] = x;
+        __syncthreads();
+    }
+    *total = part[255];
+    __syncthreads();
+    return make_int3(x.x - v.x, x.y - v.y, x.z - v.z);
+}
+__device__ __forceinline__ int3 ee_cell_counts(int n)
+{
+    return make_int3(n > 0, n, (n + kEeGroup - 1) / kEeGroup);
+}
+__global__ __launch_bounds__(256) void k_ee_scan_blocks(int64_t cells, const int *__restrict__ cnt, int3 *__restrict__ bsum)
+{
+    const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    int3 total;
+    (void)ee_scan256(ee_cell_counts(q < cells ? cnt[q] : 0), &total);
+    if (threadIdx.x == 0) bsum[blockIdx.x] = total;
+}
+// block sums to exclusive block offsets; bsum[nb] receives the totals
+__global__ __launch_bounds__(256) void k_ee_scan_top(int64_t nb, int3 *__restrict__ bsum)
+{
+    constexpr int kRun = 16;  // consecutive blocks per thread
+    int3 base = make_int3(0, 0, 0);
+    for (int64_t b0 = 0; b0 < nb; b0 += 256 * kRun) {
+        const int64_t first = b0 + (int64_t)threadIdx.x * kRun, last = min(first + kRun, nb);
+        int3 run = make_int3(0, 0, 0), total;
+        for (int64_t b = first; b < last; b++) {
+            const int3 v = bsum[b];
+            run = make_int3(run.x + v.x, run.y + v.y, run.z + v.z);
+        }
+        int3 x = ee_scan256(run, &total);
+        x = make_int3(base.x + x.x, base.y + x.y, base.z + x.z);
+        for (int64_t b = first; b < last; b++) {
+            const int3 v = bsum[b];
+            bsum[b] = x;
+            x = make_int3(x.x + v.x, x.y + v.y, x.z + v.z);
+        }
+        base = make_int3(base.x + total.x, base.y + total.y, base.z + total.z);
+    }
+    if (threadIdx.x == 0) bsum[nb] = base;
+}
+// per non-empty cell: its row's cell, first group, and the groups; cnt becomes
+// the cell's first place in order
+__global__ __launch_bounds__(256) void k_ee_scan_rows(int64_t cells, int *__restrict__ cnt, const int3 *__restrict__ bsum,
+                                                      int *__restrict__ rowcell, int *__restrict__ rowgrp,
+                                                      int4 *__restrict__ grp)
+{
+    const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int n = q < cells ? cnt[q] : 0;
+    int3 total;
+    const int3 x = ee_scan256(ee_cell_counts(n), &total), b = bsum[blockIdx.x];
+    const int row = b.x + x.x, first = b.y + x.y, g = b.z + x.z;
+    if (q < cells) cnt[q] = first;
+    if (!n) return;
+    rowcell[row] = (int)q;
+    rowgrp[row] = g;
+    for (int k = 0; k * kEeGroup < n; k++)
+        grp[g + k] = make_int4(row, first + k * kEeGroup, min(kEeGroup, n - k * kEeGroup), 0);
+}
+__global__ __launch_bounds__(256) void k_ee_place(int64_t n, const int *__restrict__ cell, const int *__restrict__ rank,
+                                                  const int *__restrict__ cnt, int *__restrict__ order)
+{
+    const int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (f < n) order[cnt[cell[f]] + rank[f]] = (int)f;
+}
+
 // P3..P6 of n stored pairs (k1, ka) at f, one thread per element (i1 i2 ia ib):
 //   P3/P4: k3 over k, k4 = k1 + k3 - ka, A from calc_A(k1, k4, k3, ka),
 //     P3 += sum_{i4 i3} A1[(i1 i4),(i3 ia)] (1-f3) f4 conj(A2[(i2 i4),(i3 ib)]),
@@ -907,6 +1340,104 @@ void launch_ee_P(dmd_scatt *h, int64_t n, const uint64_t *d1, const uint64_t *d2
                            s2);
 }
 
+// Scratch of the grouped path, held over the chunks of one call.
+struct EeGroups {
+    char *mem = nullptr;  // one allocation for the arrays below
+    int *cnt = nullptr, *cell = nullptr, *rank = nullptr, *order = nullptr, *rowcell = nullptr, *rowgrp = nullptr;
+    int3 *bsum = nullptr;
+    int4 *grp = nullptr;
+    double *tab = nullptr;
+    int64_t tab_rows = 0;
+    std::vector<int> h_rowgrp;
+    ~EeGroups()
+    {
+        dfree(mem);
+        dfree(tab);
+    }
+};
+constexpr int64_t kEeCells = 1ll << 26;     // mesh cells the grouping counts over (256 MiB)
+constexpr int64_t kEeTabBytes = 192ll << 20;  // (q, k3) table held at once: it stays in the last-level cache
+// Pairs per distinct q from which the grouped path is taken.  A table row
+// costs its nk entries' overlaps and products whatever share of them a pair's
+// window keeps.  12^3 mesh: at 4.0 pairs per q 2.1 ms grouped and 1.85 per
+// pair, at 8.0 2.4 and 3.3, at 16 3.3 and 6.1.  Fewer pairs than that per k
+// point are not counted by q at all (the count costs 0.13 ms).
+constexpr int64_t kEeShare = 6;
+
+// P1, P2 of the chunk's n pairs (file order) grouped by q; *done = false when
+// the pairs are too scattered over q for it (nothing has been written then).
+template <int NB>
+int launch_ee_groups(dmd_scatt *h, int64_t n, int64_t chunk, const uint64_t *d1, const uint64_t *d2, const EeArgs &a,
+                     const EimpConst &c, EeGroups &s, double2 *s1, double2 *s2, bool *done)
+{
+    *done = false;
+    const int64_t cells = (int64_t)a.m0 * a.m1 * a.m2;
+    const int64_t nb = (cells + 255) / 256, ntile = (a.nk + kEeTile - 1) / kEeTile;
+    int rc;
+    if (!s.mem) {
+        const size_t most = (size_t)std::min(chunk, cells);
+        size_t bytes = 0;
+        auto take = [&](size_t n) {  // 16-byte aligned places
+            const size_t at = bytes;
+            bytes += (n + 15) / 16 * 16;
+            return at;
+        };
+        const size_t o_cnt = take((size_t)cells * 4), o_bsum = take(((size_t)nb + 1) * sizeof(int3)),
+                     o_cell = take((size_t)chunk * 4), o_rank = take((size_t)chunk * 4),
+                     o_order = take((size_t)chunk * 4), o_rowcell = take(most * 4), o_rowgrp = take(most * 4),
+                     o_grp = take((size_t)chunk * sizeof(int4));
+        if ((rc = dalloc_t(&s.mem, bytes, "e-e pair groups"))) return rc;
+        s.cnt = (int *)(s.mem + o_cnt);
+        s.bsum = (int3 *)(s.mem + o_bsum);
+        s.cell = (int *)(s.mem + o_cell);
+        s.rank = (int *)(s.mem + o_rank);
+        s.order = (int *)(s.mem + o_order);
+        s.rowcell = (int *)(s.mem + o_rowcell);
+        s.rowgrp = (int *)(s.mem + o_rowgrp);
+        s.grp = (int4 *)(s.mem + o_grp);
+    }
+    hipLaunchKernelGGL(k_fill_int, dim3(nblk(cells, 256)), dim3(256), 0, h->st, cells, s.cnt, 0);
+    hipLaunchKernelGGL(k_ee_qcell, dim3(nblk(n, 256)), dim3(256), 0, h->st, n, d1, d2, a, s.cnt, s.cell, s.rank);
+    hipLaunchKernelGGL(k_ee_scan_blocks, dim3((unsigned)nb), dim3(256), 0, h->st, cells, s.cnt, s.bsum);
+    hipLaunchKernelGGL(k_ee_scan_top, dim3(1), dim3(256), 0, h->st, nb, s.bsum);
+    hipLaunchKernelGGL(k_ee_scan_rows, dim3((unsigned)nb), dim3(256), 0, h->st, cells, s.cnt, s.bsum, s.rowcell,
+                       s.rowgrp, s.grp);
+    hipLaunchKernelGGL(k_ee_place, dim3(nblk(n, 256)), dim3(256), 0, h->st, n, s.cell, s.rank, s.cnt, s.order);
+    DMD_HIP(hipGetLastError());
+    int3 tot;
+    DMD_HIP(hipMemcpyAsync(&tot, s.bsum + nb, sizeof(tot), hipMemcpyDeviceToHost, h->st));
+    DMD_HIP(hipStreamSynchronize(h->st));
+    const int64_t rows = tot.x, groups = tot.z;
+    if (n < kEeShare * rows) return DMD_OK;
+    const size_t row_words = (size_t)ntile * EeTab<NB>::F * kEeTile;
+    const int64_t want = std::min(rows, std::max<int64_t>(1, kEeTabBytes / (int64_t)(row_words * 8)));
+    if (want > s.tab_rows) {
+        dfree(s.tab);
+        s.tab = nullptr;
+        s.tab_rows = 0;
+        if ((rc = dalloc_t(&s.tab, row_words * (size_t)want, "e-e table"))) return rc;
+        s.tab_rows = want;
+    }
+    s.h_rowgrp.resize((size_t)rows);
+    if (rows > want) {
+        DMD_HIP(hipMemcpyAsync(s.h_rowgrp.data(), s.rowgrp, (size_t)rows * 4, hipMemcpyDeviceToHost, h->st));
+        DMD_HIP(hipStreamSynchronize(h->st));
+    } else {
+        s.h_rowgrp[0] = 0;
+    }
+    for (int64_t r0 = 0; r0 < rows; r0 += want) {
+        const int64_t r1 = std::min(rows, r0 + want);
+        const int64_t g0 = s.h_rowgrp[(size_t)r0], g1 = r1 < rows ? s.h_rowgrp[(size_t)r1] : groups;
+        hipLaunchKernelGGL(k_ee_qtab<NB>, dim3(nblk((r1 - r0) * ntile * kEeTile, 256)), dim3(256), 0, h->st, r1 - r0,
+                           ntile, s.rowcell + r0, a, s.tab);
+        hipLaunchKernelGGL(k_ee_group<NB>, dim3((unsigned)(g1 - g0)), dim3(64 * kEeGroup), 0, h->st, s.grp + g0, (int)r0,
+                           ntile, s.order, d1, d2, a, c, s.tab, s1, s2);
+    }
+    DMD_HIP(hipGetLastError());
+    *done = true;
+    return DMD_OK;
+}
+
 // The fold of scale x P_ee into P of every stored pair (add = 0: set), chunked.
 // vq_pair_host: v(k1 - k2) of every stored pair (or null: a.vq_cell / closed form).
 // rows (device, 2 nk nb^2 complex, zeroed): the chunks' dP go into the
@@ -928,6 +1459,12 @@ int ee_fold(dmd_scatt *h, const uint64_t *k1st, const uint64_t *k2nd, EeArgs a, 
         release();
         return rc;
     }
+    // Lindblad form without exchange: pairs grouped by q (DMD_EE_FORMS: the
+    // ungrouped kernels, for comparison)
+    const int64_t cells = (int64_t)a.m0 * a.m1 * a.m2;
+    bool grouped = h->nb <= 2 && c.m.lindblad && !c.m.exchange && cells <= kEeCells &&
+                   h->np >= kEeShare * std::min(h->nk, cells) && !std::getenv("DMD_EE_FORMS");
+    EeGroups groups;
     hipError_t e = hipSuccess;
     for (int64_t first = 0; first < h->np && e == hipSuccess && rc == DMD_OK; first += chunk) {
         const int64_t n = std::min(chunk, h->np - first);
@@ -937,7 +1474,17 @@ int ee_fold(dmd_scatt *h, const uint64_t *k1st, const uint64_t *k2nd, EeArgs a, 
             e = hipMemcpyAsync(dvq, vq_pair_host->data() + first, (size_t)n * 8, hipMemcpyHostToDevice, h->st);
         if (e != hipSuccess) break;
         a.vq_pair = vq_pair_host ? dvq : nullptr;
-        switch (h->nb) {
+        bool done = false;
+        if (grouped) {
+            rc = h->nb == 1 ? launch_ee_groups<1>(h, n, chunk, d1, d2, a, c, groups, s1, s2, &done)
+                            : launch_ee_groups<2>(h, n, chunk, d1, d2, a, c, groups, s1, s2, &done);
+            if (rc == DMD_ERR_NOMEM) {  // no room for the table: the ungrouped kernel
+                grouped = false;
+                rc = DMD_OK;
+            }
+            if (rc) break;
+        }
+        if (!done) switch (h->nb) {
         case 1: launch_ee_P<1>(h, n, d1, d2, a, c, s1, s2); break;
         case 2: launch_ee_P<2>(h, n, d1, d2, a, c, s1, s2); break;
         case 3: launch_ee_P<3>(h, n, d1, d2, a, c, s1, s2); break;
