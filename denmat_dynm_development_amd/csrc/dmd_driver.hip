@@ -9,9 +9,11 @@
 // (src_v4.5.7/observable.h:301-366), evolve_driver (evolve_eph.cpp:21-32).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "dmd_internal.h"
@@ -249,6 +251,319 @@ static StageArgs stage_args(dmd_scatt *h, double dt)
     return A;
 }
 
+// ---------------------------------------------------------------------------
+// Fused stage kernels for the tile contraction's packed Hermitian rows: the
+// assembly of the scattering term, the rest of the right-hand side, the
+// integrator's combination and the rotation of the next stage's state in one
+// launch, so a stage is the contraction and one kernel.  (Apart, a stage was
+// three to five launches of 4 to 10 us each, half the time of a step of an
+// operator of a few 100 k pairs.)  A block takes whole k points, one thread
+// per element (i, j); the state's row and H(t) are staged in LDS, so every
+// phase cis((e_i - e_j) t) is formed once instead of once per product term.
+// ---------------------------------------------------------------------------
+struct PackedArgs {
+    double *hacc;         // nk x NB^2 packed rows (cleared here)
+    const double *feq;    // reduced forms: nk x 64 row sums at diag f, or null
+    double2 *rhoS;        // nk x NB^2: the state the sums were formed at; the next stage's on return
+    const double2 *eq;    // ddmdt_eq or null
+    double prefac;
+    const double *f;      // reduced forms: occupations of the split, or null
+    float2 *x32;          // reduced forms: the next contraction's operand, or null
+};
+struct StageLds {
+    double2 y[256], H[256], r[256];
+};
+// the thread's place: element (i, j) of k; live: inside the arrays
+struct StagePos {
+    int n, n2, row, ij, i, j, wi, wj;
+    int64_t k, idx;
+    bool live, win;
+};
+__device__ __forceinline__ StagePos stage_pos(const StageArgs &A)
+{
+    StagePos p;
+    p.n = A.nbd;
+    p.n2 = A.nbd * A.nbd;
+    const int rows = 256 / p.n2;
+    p.row = threadIdx.x / p.n2;
+    p.ij = threadIdx.x - p.row * p.n2;
+    p.i = p.ij / p.n;
+    p.j = p.ij - p.i * p.n;
+    p.wi = p.i - A.b0;
+    p.wj = p.j - A.b0;
+    p.k = (int64_t)blockIdx.x * rows + p.row;
+    p.idx = p.k * p.n2 + p.ij;
+    p.live = p.row < rows && p.k < A.nk;
+    p.win = p.live && p.wi >= 0 && p.wi < A.nb && p.wj >= 0 && p.wj < A.nb;
+    return p;
+}
+__device__ __forceinline__ double2 stage_phase(const StageArgs &A, const StagePos &p, double t)
+{
+    return ccis((A.edm[p.k * p.n + p.i] - A.edm[p.k * p.n + p.j]) * t);
+}
+
+// f(t, yin) at the thread's element.  Called by every thread of the block;
+// clears the block's packed rows.  ph: cis((e_i - e_j) t) where it was needed.
+template <int NB>
+__device__ __forceinline__ double2 stage_slope(const StageArgs &A, const PackedArgs &Q, const StagePos &p,
+                                               const double2 *yin, double t, StageLds &L, double2 &ph)
+{
+    constexpr int NB2 = NB * NB;
+    const int tid = threadIdx.x, base = tid - p.ij;
+    const bool coh = A.coh && !A.semic;
+    double2 y = make_double2(0, 0), Ht = make_double2(0, 0), d = make_double2(0, 0);
+    ph = make_double2(1.0, 0.0);
+    const int m = p.wi * NB + p.wj;
+    if (p.live) {
+        y = yin[p.idx];
+        if (p.i != p.j && (A.expt || (!A.schrod && (Q.eq || (coh && A.H))))) ph = stage_phase(A, p, t);
+        if (coh && A.H) {
+            Ht = herm_up_rt(A.H + p.k * p.n2, p.n, p.i, p.j);
+            if (A.schrod) {
+                if (p.i == p.j) Ht.x += A.edm[p.k * p.n + p.i];
+            } else if (p.i != p.j) {
+                Ht = cmul(Ht, ph);
+            }
+        }
+    }
+    if (p.win) {
+        const double *h = Q.hacc + p.k * NB2;
+        if constexpr (NB == 2) {
+            if (p.wi == p.wj) d = make_double2(h[p.wi], 0.0);
+            else d = make_double2(h[2], p.wi < p.wj ? h[3] : -h[3]);
+        } else {
+            if (p.wi == p.wj) d = make_double2(h[5 * p.wi], 0.0);
+            else if (p.wi < p.wj) d = make_double2(h[m], h[4 * p.wj + p.wi]);
+            else d = make_double2(h[4 * p.wj + p.wi], -h[m]);
+            if (Q.feq) L.r[p.row * NB2 + m] = Q.rhoS[p.k * NB2 + m];
+        }
+    }
+    L.y[tid] = y;
+    L.H[tid] = Ht;
+    __syncthreads();  // every packed row of the block is read
+    if (p.live && p.ij < NB2) Q.hacc[p.k * NB2 + p.ij] = 0.0;
+    double2 kv = make_double2(0, 0);
+    if (!p.live || (A.semic && p.i != p.j)) return kv;
+    if (coh) {
+        if (A.H) {
+            double2 yh = make_double2(0, 0), hy = make_double2(0, 0);
+            for (int q = 0; q < p.n; q++) {
+                yh = cadd(yh, cmul(L.y[base + p.i * p.n + q], L.H[base + q * p.n + p.j]));
+                hy = cadd(hy, cmul(L.H[base + p.i * p.n + q], L.y[base + q * p.n + p.j]));
+            }
+            const double2 c = csub(hy, yh);
+            kv = make_double2(c.y, -c.x);  // times -i
+        } else {  // Schroedinger picture without H
+            const double w = A.edm[p.k * p.n + p.i] - A.edm[p.k * p.n + p.j];
+            kv = make_double2(w * y.y, -(w * y.x));
+        }
+    }
+    if (p.win) {
+        if constexpr (NB == 4) {
+            if (Q.feq) {  // C_eq + C_eq^+, C_eq = (1 - rho) F1eq - F2eq rho
+                const double *F = Q.feq + p.k * 64;
+                const double2 *rk = L.r + p.row * NB2;
+                const double2 xij = c_elem(F, rk, nullptr, p.wi, p.wj), xji = c_elem(F, rk, nullptr, p.wj, p.wi);
+                d = cadd(d, cadd(xij, cconj(xji)));
+            }
+        }
+        d = make_double2(d.x * (Q.prefac * 0.5), d.y * (Q.prefac * 0.5));
+        if (A.expt && p.i != p.j) d = cmul(d, ph);
+        if (Q.eq) {
+            double2 q = Q.eq[p.k * NB2 + m];
+            if (p.i != p.j && !A.schrod) q = cmul(q, ph);
+            d = csub(d, q);
+        }
+        kv = cadd(kv, d);
+    }
+    if (A.ph_tau_inv != 0.0 && p.i >= A.ph_b0 && p.i < A.ph_b1 && p.j >= A.ph_b0 && p.j < A.ph_b1) {
+        double2 q = y;
+        if (p.i == p.j) q.x -= A.ph_feq[p.k * p.n + p.i];
+        kv = csub(kv, make_double2(q.x * A.ph_tau_inv, q.y * A.ph_tau_inv));
+    }
+    return kv;
+}
+
+// the window of the next stage's state v in the Schroedinger picture, ph the
+// phase cis((e_i - e_j) t) at its time
+template <int NB>
+__device__ __forceinline__ void stage_rotate(const StageArgs &A, const PackedArgs &Q, const StagePos &p, double2 v,
+                                             double2 ph)
+{
+    if (!p.win) return;
+    if (A.expt && p.wi != p.wj) v = cmulc(v, ph);
+    if (A.fsub && p.wi == p.wj) v.x -= A.fsub[p.k * NB + p.wi];
+    if (A.semic && p.wi != p.wj) v = make_double2(0.0, 0.0);
+    const int64_t q = p.k * (NB * NB) + p.wi * NB + p.wj;
+    Q.rhoS[q] = v;
+    if (Q.x32) {
+        if (Q.f && p.wi == p.wj) v.x -= Q.f[p.k * NB + p.wi];
+        Q.x32[q] = make_float2((float)v.x, (float)v.y);
+    }
+}
+
+// RK4 stages 0..2 on packed rows (k_rk_stage with the assembly)
+template <int NB>
+__global__ __launch_bounds__(256) void k_stage_rk4(StageArgs A, PackedArgs Q, int s, const double2 *__restrict__ yin,
+                                                   const double2 *__restrict__ y0, double2 *__restrict__ acc,
+                                                   double2 *__restrict__ yout)
+{
+    __shared__ StageLds L;
+    const double a_s[4] = { 0.0, 0.5, 0.5, 1.0 }, w_s[4] = { 1.0, 2.0, 2.0, 1.0 };
+    const StagePos p = stage_pos(A);
+    double2 ph;
+    const double2 kv = stage_slope<NB>(A, Q, p, yin, clock_t_at(A.clk, a_s[s]), L, ph);
+    if (!p.live) return;
+    acc[p.idx] = s == 0 ? kv : cadd(acc[p.idx], make_double2(w_s[s] * kv.x, w_s[s] * kv.y));
+    const double c = a_s[s + 1] * A.dt;
+    const double2 y = make_double2(y0[p.idx].x + c * kv.x, y0[p.idx].y + c * kv.y);
+    yout[p.idx] = y;
+    if (s != 1 && A.expt && p.win && p.i != p.j) ph = stage_phase(A, p, clock_t_at(A.clk, a_s[s + 1]));
+    stage_rotate<NB>(A, Q, p, y, ph);
+}
+
+// RK4 stage 3 on packed rows: y = y0 + dt/6 (acc + kv), Hermitized, into ynew
+// (y0 itself is allowed), rotated at the next step's first stage; the last
+// block to end advances the clock (tick).
+template <int NB>
+__global__ __launch_bounds__(256) void k_stage_rk4_final(StageArgs A, PackedArgs Q, const double2 *__restrict__ yin,
+                                                         const double2 *y0, const double2 *__restrict__ acc,
+                                                         double2 *ynew, DClock *tick)
+{
+    __shared__ StageLds L;
+    const StagePos p = stage_pos(A);
+    double2 ph;
+    const double2 kv = stage_slope<NB>(A, Q, p, yin, clock_t_at(A.clk, 1.0), L, ph);
+    const double tn = (A.clk->t0 + (double)(A.clk->step + 1) * A.clk->dt) + 0.0 * A.clk->dt;
+    const double c = A.dt / 6.0;
+    double2 v = make_double2(0, 0);
+    if (p.live) {
+        const double2 a = cadd(acc[p.idx], kv);
+        v = make_double2(y0[p.idx].x + c * a.x, y0[p.idx].y + c * a.y);
+    }
+    __syncthreads();  // the staged rows are read
+    L.y[threadIdx.x] = v;
+    __syncthreads();
+    if (p.live) {
+        const double2 o = L.y[threadIdx.x - p.ij + p.j * p.n + p.i];
+        if (p.i == p.j) v.y = 0.0;
+        else v = make_double2(0.5 * (v.x + o.x), 0.5 * (v.y - o.y));
+        ynew[p.idx] = v;
+        if (A.expt && p.win && p.i != p.j) ph = stage_phase(A, p, tn);
+        stage_rotate<NB>(A, Q, p, v, ph);
+    }
+    if (!tick) return;
+    __syncthreads();  // the block has read the clock
+    if (threadIdx.x == 0) {
+        __threadfence();
+        if (atomicAdd((unsigned long long *)&tick->pad, 1ull) == gridDim.x - 1) {
+            tick->pad = 0;
+            tick->step += 1;
+        }
+    }
+}
+
+struct Coef6 {
+    double c[6];
+};
+struct Ptr6 {
+    const double2 *p[6];
+};
+
+// A stage on packed rows at time a: kout = f; with m > 0 also the next stage's
+// state ynext = y0 + h sum_j<m c_j k_j (k_{m-1} = this slope), rotated at time
+// a_next.  yin may be ynext.
+template <int NB>
+__global__ __launch_bounds__(256) void k_stage_comb(StageArgs A, PackedArgs Q, double a, double a_next,
+                                                    const double2 *yin, const double2 *__restrict__ y0, double h, int m,
+                                                    Coef6 c, Ptr6 k, double2 *__restrict__ kout, double2 *ynext)
+{
+    __shared__ StageLds L;
+    const StagePos p = stage_pos(A);
+    double2 ph;
+    const double2 kv = stage_slope<NB>(A, Q, p, yin, clock_t_at(A.clk, a), L, ph);
+    if (!p.live) return;
+    kout[p.idx] = kv;
+    if (m == 0) return;
+    double2 s = make_double2(0, 0);
+    for (int j = 0; j < m; j++) {
+        const double2 v = j == m - 1 ? kv : k.p[j][p.idx];
+        s.x += c.c[j] * v.x;
+        s.y += c.c[j] * v.y;
+    }
+    const double2 y = make_double2(y0[p.idx].x + h * s.x, y0[p.idx].y + h * s.y);
+    ynext[p.idx] = y;
+    if (A.expt && p.win && p.i != p.j) ph = stage_phase(A, p, clock_t_at(A.clk, a_next));
+    stage_rotate<NB>(A, Q, p, y, ph);
+}
+
+// The last rkf45 stage on packed rows: k_6 stays in registers, ynew = y0 + h sum
+// b_j k_j, and the block's max of |h sum e_j k_j| / (eps_abs + eps_rel |ynew|).
+template <int NB>
+__global__ __launch_bounds__(256) void k_stage_rkf_final(StageArgs A, PackedArgs Q, double a,
+                                                         const double2 *__restrict__ yin,
+                                                         const double2 *__restrict__ y0, double h, Coef6 b, Coef6 e,
+                                                         Ptr6 k, double eps_abs, double eps_rel,
+                                                         double2 *__restrict__ ynew, double *__restrict__ part)
+{
+    __shared__ StageLds L;
+    __shared__ double red[256];
+    const StagePos p = stage_pos(A);
+    double2 ph;
+    const double2 kv = stage_slope<NB>(A, Q, p, yin, clock_t_at(A.clk, a), L, ph);
+    double r = 0.0;
+    if (p.live) {
+        double2 s = make_double2(0, 0), q = make_double2(0, 0);
+#pragma unroll
+        for (int j = 0; j < 6; j++) {
+            const double2 v = j == 5 ? kv : k.p[j][p.idx];
+            s.x += b.c[j] * v.x; s.y += b.c[j] * v.y;
+            q.x += e.c[j] * v.x; q.y += e.c[j] * v.y;
+        }
+        const double2 y = make_double2(y0[p.idx].x + h * s.x, y0[p.idx].y + h * s.y);
+        ynew[p.idx] = y;
+        r = fmax(fabs(h * q.x) / (eps_abs + eps_rel * fabs(y.x)), fabs(h * q.y) / (eps_abs + eps_rel * fabs(y.y)));
+    }
+    red[threadIdx.x] = r;
+    __syncthreads();
+    for (int w = 128; w > 0; w >>= 1) {
+        if ((int)threadIdx.x < w) red[threadIdx.x] = fmax(red[threadIdx.x], red[threadIdx.x + w]);
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) part[blockIdx.x] = red[0];
+}
+
+// the fused stages run where the contraction leaves packed rows
+static PackedArgs packed_args(dmd_scatt *h)
+{
+    const bool red = h->precision != DMD_PREC_FP64 && !h->linear;
+    PackedArgs Q;
+    Q.hacc = h->nb == 4 ? h->d_hacc16 : h->d_acc_herm;
+    Q.feq = red ? h->d_feq : nullptr;
+    Q.rhoS = h->d_rhoS;
+    Q.eq = h->has_eq ? h->d_eq : nullptr;
+    Q.prefac = h->prefac;
+    Q.f = red ? h->d_fsplit : nullptr;
+    Q.x32 = red ? h->d_x32 : nullptr;
+    return Q;
+}
+static unsigned stage_blocks(const dmd_scatt *h)
+{
+    return nblk(h->nk, 256 / (h->nbd * h->nbd));
+}
+// the first stage's operand: the window of y at stage a, and the reduced forms' drho
+static int packed_begin(dmd_scatt *h, const double2 *y, double a)
+{
+    int rc;
+    if ((rc = launch_rotate(h, y, nullptr, h->nbd, h->b0, a, h->semiclassical))) return rc;
+    return h->precision != DMD_PREC_FP64 && !h->linear ? launch_split_x(h) : DMD_OK;
+}
+#define DMD_STAGE(KERNEL, ...)                                                                                       \
+    do {                                                                                                             \
+        if (h->nb == 2) hipLaunchKernelGGL(KERNEL<2>, dim3(stage_blocks(h)), dim3(256), 0, h->st, __VA_ARGS__);      \
+        else hipLaunchKernelGGL(KERNEL<4>, dim3(stage_blocks(h)), dim3(256), 0, h->st, __VA_ARGS__);                 \
+    } while (0)
+
 static int ensure_rk(dmd_scatt *h)
 {
     const int64_t n = h->nk * (int64_t)h->nbd * h->nbd;
@@ -265,12 +580,46 @@ static int ensure_rk(dmd_scatt *h)
     return DMD_OK;
 }
 
+// the report series of a run, kept between runs (grown by doubling)
+static int ensure_obs(dmd_scatt *h, int64_t n)
+{
+    if (h->obs_series_cap >= n) return DMD_OK;
+    dfree(h->d_obs_series);
+    h->d_obs_series = nullptr;
+    const int64_t cap = std::max<int64_t>(n, std::max<int64_t>(256, 2 * h->obs_series_cap));
+    h->obs_series_cap = 0;
+    int rc;
+    if ((rc = dalloc_t(&h->d_obs_series, (size_t)cap, "obs series"))) return rc;
+    h->obs_series_cap = cap;
+    return DMD_OK;
+}
+
 static int launch_obs(dmd_scatt *h, const double2 *y, double *out, int idx)
 {
     unsigned nb = nblk(h->nk, 256);
     hipLaunchKernelGGL(k_obs_partial, dim3(nb), dim3(256), 0, h->st, h->nk, h->nbd, h->obs_i0, h->obs_i1, h->d_s,
                        h->d_edm, h->d_f, y, h->d_clk, h->schrodinger ? 0 : 1, h->d_part);
     hipLaunchKernelGGL(k_obs_final, dim3(1), dim3(256), 0, h->st, (int)nb, h->d_part, h->obs_prefac, out, idx);
+    DMD_HIP(hipGetLastError());
+    return DMD_OK;
+}
+
+int rk4_packed_begin(dmd_scatt *h, const double2 *y, double t0, double dt, int64_t j)
+{
+    int rc;
+    if ((rc = set_clock(h, t0, dt, j))) return rc;
+    return packed_begin(h, y, 0.0);
+}
+int rk4_packed_step(dmd_scatt *h, double dt, const double2 *y, double2 *const Y[3], double2 *acc, double2 *ynext)
+{
+    const StageArgs A = stage_args(h, dt);
+    const PackedArgs Q = packed_args(h);
+    int rc;
+    for (int s = 0; s < 4; s++) {
+        if ((rc = launch_packed_sums(h))) return rc;
+        if (s < 3) DMD_STAGE(k_stage_rk4, A, Q, s, s ? Y[s - 1] : y, y, acc, Y[s]);
+        else DMD_STAGE(k_stage_rk4_final, A, Q, Y[2], y, acc, ynext, h->d_clk);
+    }
     DMD_HIP(hipGetLastError());
     return DMD_OK;
 }
@@ -287,6 +636,10 @@ static int launch_step(dmd_scatt *h, const StageArgs &A, int64_t it = 0, double 
     double2 *yin[4] = { h->d_y0, h->d_ya, h->d_yb, h->d_ya };
     double2 *yout[3] = { h->d_ya, h->d_yb, h->d_ya };
     int rc;
+    if (packed_rows(h) && !h->rhs_hook) {
+        double2 *const Y[3] = { yout[0], yout[1], yout[2] };
+        return rk4_packed_step(h, A.dt, h->d_y0, Y, h->d_acc, h->d_y0);
+    }
     for (int s = 0; s < 4; s++) {
         if (h->rhs_hook && (rc = run_rhs_hook(h, t0 + ((double)it + a_s[s]) * dt, yin[s]))) return rc;
         if ((rc = launch_contract(h, false, a_s[s], h->d_w))) return rc;
@@ -351,10 +704,20 @@ extern "C" int dmd_scatt_evolve_driver(dmd_scatt *h, double t, const double *dm,
     if ((rc = tiles4_prepare(h))) return rc;
     if ((rc = set_clock(h, t, 0.0, 0))) return rc;
     if ((rc = launch_rotate(h, in, in1, h->nbd, h->b0, 0.0))) return rc;
-    if ((rc = launch_contract(h, dm1 != nullptr, 0.0, h->d_w))) return rc;
     double2 *out = is_device_ptr(ddmdt) ? (double2 *)ddmdt : h->d_out;
     int64_t n = h->nk * (int64_t)h->nbd * h->nbd;
-    hipLaunchKernelGGL(k_expand, dim3(nblk(n, 256)), dim3(256), 0, h->st, h->nk, h->nb, h->nbd, h->b0, h->d_w, out);
+    if (packed_rows(h)) {  // the scattering term alone, expanded, as a stage's slope
+        if (h->precision != DMD_PREC_FP64 && !h->linear && (rc = launch_split_x(h))) return rc;
+        if ((rc = launch_packed_sums(h, dm1 != nullptr))) return rc;
+        StageArgs A = stage_args(h, 0.0);
+        A.coh = 0;
+        A.semic = 0;
+        A.ph_tau_inv = 0.0;
+        DMD_STAGE(k_stage_comb, A, packed_args(h), 0.0, 0.0, in, in, 0.0, 0, Coef6{}, Ptr6{}, out, (double2 *)nullptr);
+    } else {
+        if ((rc = launch_contract(h, dm1 != nullptr, 0.0, h->d_w))) return rc;
+        hipLaunchKernelGGL(k_expand, dim3(nblk(n, 256)), dim3(256), 0, h->st, h->nk, h->nb, h->nbd, h->b0, h->d_w, out);
+    }
     DMD_HIP(hipGetLastError());
     if (out == h->d_out && (rc = from_device(h, ddmdt, h->d_out, bytes))) return rc;
     DMD_HIP(hipStreamSynchronize(h->st));
@@ -419,18 +782,25 @@ extern "C" int dmd_scatt_integrate_rk4(dmd_scatt *h, double t0, double dt, int64
     if ((rc = ensure_rk(h))) return rc;
     if ((rc = tiles4_prepare(h))) return rc;
     const int64_t nobs = want_obs ? n_steps / report_every + 1 : 0;
-    double *d_obs = nullptr;
-    if (nobs && (rc = dalloc_t(&d_obs, nobs, "obs series"))) return rc;
-    struct Guard { double *p; ~Guard() { dfree(p); } } guard{ d_obs };
+    if (nobs && (rc = ensure_obs(h, nobs))) return rc;
+    double *d_obs = h->d_obs_series;
     const size_t n = (size_t)h->nk * h->nbd * h->nbd;
     if ((rc = to_device(h, h->d_y0, rho, n * 16))) return rc;
     if ((rc = set_clock(h, t0, dt, 0))) return rc;
     StageArgs A = stage_args(h, dt);
-    if ((rc = launch_rotate(h, h->d_y0, nullptr, h->nbd, h->b0, 0.0, h->semiclassical))) return rc;
+    const bool packed = packed_rows(h) && !h->rhs_hook;
+    if ((rc = packed ? packed_begin(h, h->d_y0, 0.0)
+                     : launch_rotate(h, h->d_y0, nullptr, h->nbd, h->b0, 0.0, h->semiclassical)))
+        return rc;
     int iobs = 0;
     if (want_obs && (rc = launch_obs(h, h->d_y0, d_obs, iobs++))) return rc;
+    // The eight launches of a packed step go to the stream as they are: each
+    // replay of a captured step cost a gap of 8 us and the capture itself 50 us
+    // (2 steps of 1.4 k pairs 183 us captured, 128 us not; 20 of 0.96 M pairs
+    // 6.98 and 6.89 ms).  The other forms' steps (14 launches) are captured;
+    // DMD_GRAPH=0 launches them too.
     const char *env = std::getenv("DMD_GRAPH");
-    const bool use_graph = !(env && env[0] == '0') && n_steps > 1 && !h->rhs_hook;
+    const bool use_graph = !packed && !(env && env[0] == '0') && n_steps > 1 && !h->rhs_hook;
     hipGraphExec_t exec = nullptr;
     if (use_graph) {
         hipGraph_t graph = nullptr;
@@ -443,21 +813,15 @@ extern "C" int dmd_scatt_integrate_rk4(dmd_scatt *h, double t0, double dt, int64
         (void)hipGraphDestroy(graph);
         if (e != hipSuccess) return fail(DMD_ERR_HIP, std::string("graph instantiate: ") + hipGetErrorString(e));
     }
+    struct Guard { hipStream_t st; hipGraphExec_t e; ~Guard() { if (e) { (void)hipStreamSynchronize(st); (void)hipGraphExecDestroy(e); } } } guard{ h->st, exec };
     for (int64_t it = 0; it < n_steps; it++) {
         if (exec) {
-            hipError_t e = hipGraphLaunch(exec, h->st);
-            if (e != hipSuccess) { (void)hipGraphExecDestroy(exec); return fail(DMD_ERR_HIP, hipGetErrorString(e)); }
+            DMD_HIP(hipGraphLaunch(exec, h->st));
         } else if ((rc = launch_step(h, A, it, t0, dt))) {
             return rc;
         }
-        if (want_obs && (it + 1) % report_every == 0 && (rc = launch_obs(h, h->d_y0, d_obs, iobs++))) {
-            if (exec) (void)hipGraphExecDestroy(exec);
-            return rc;
-        }
+        if (want_obs && (it + 1) % report_every == 0 && (rc = launch_obs(h, h->d_y0, d_obs, iobs++))) return rc;
     }
-    hipError_t e = hipStreamSynchronize(h->st);
-    if (exec) (void)hipGraphExecDestroy(exec);
-    if (e != hipSuccess) return fail(DMD_ERR_HIP, hipGetErrorString(e));
     if ((rc = from_device(h, rho, h->d_y0, n * 16))) return rc;
     if (nobs) DMD_HIP(hipMemcpyAsync(obs_out, d_obs, nobs * 8, hipMemcpyDeviceToHost, h->st));
     DMD_HIP(hipStreamSynchronize(h->st));
@@ -661,13 +1025,6 @@ extern "C" int dmd_scatt_integrate_rk4_batched(dmd_scatt *h, int B, double t0, d
 // ---------------------------------------------------------------------------
 namespace dmd {
 
-struct Coef6 {
-    double c[6];
-};
-struct Ptr6 {
-    const double2 *p[6];
-};
-
 // kout = f(t + a h, y): the full right-hand side from the window ddm w
 __global__ void k_rhs_full(StageArgs A, const double2 *__restrict__ y, const double2 *__restrict__ w, double a,
                            double2 *__restrict__ kout)
@@ -768,8 +1125,16 @@ static int ensure_adaptive(dmd_scatt *h)
     dfree(h->d_ad); dfree(h->d_adpart);
     h->d_ad = nullptr; h->d_adpart = nullptr;
     h->ad_cap = 0;
+    if (!h->h_ratio) {
+        const hipError_t e = hipHostMalloc((void **)&h->h_ratio, sizeof(double), hipHostMallocDefault);
+        if (e != hipSuccess) {
+            h->h_ratio = nullptr;
+            return fail(DMD_ERR_NOMEM, std::string("pinned error ratio: ") + hipGetErrorString(e));
+        }
+    }
     if ((rc = dalloc_t(&h->d_ad, (size_t)9 * n, "adaptive integrator states"))) return rc;
-    if ((rc = dalloc_t(&h->d_adpart, (size_t)nblk(n, 256) + 1, "error partials"))) return rc;
+    // one per block of k_rkf_final or of the fused stage (whole k points per block)
+    if ((rc = dalloc_t(&h->d_adpart, (size_t)std::max(nblk(n, 256), stage_blocks(h)) + 1, "error partials"))) return rc;
     h->ad_cap = n;
     return DMD_OK;
 }
@@ -794,6 +1159,12 @@ static int full_rhs(dmd_scatt *h, const StageArgs &A, const double2 *y, double a
     if (h->rhs_hook &&
         (rc = run_rhs_hook(h, h->h_clk.t0 + ((double)h->h_clk.step + a) * h->h_clk.dt, y)))
         return rc;
+    if (packed_rows(h)) {
+        if ((rc = packed_begin(h, y, a)) || (rc = launch_packed_sums(h))) return rc;
+        DMD_STAGE(k_stage_comb, A, packed_args(h), a, a, y, y, 0.0, 0, Coef6{}, Ptr6{}, kout, (double2 *)nullptr);
+        DMD_HIP(hipGetLastError());
+        return DMD_OK;
+    }
     if ((rc = launch_rotate(h, y, nullptr, h->nbd, h->b0, a, h->semiclassical))) return rc;
     if ((rc = launch_contract(h, false, a, h->d_w))) return rc;
     const int64_t n = h->nk * (int64_t)h->nbd * h->nbd;
@@ -803,7 +1174,8 @@ static int full_rhs(dmd_scatt *h, const StageArgs &A, const double2 *y, double a
 }
 
 // one RKF45 attempt of size hs from (t, y0): ynew and the error ratio
-static int rkf45_attempt(dmd_scatt *h, double t, double hs, double eps_abs, double eps_rel, double *ratio)
+static int rkf45_attempt(dmd_scatt *h, double t, double hs, double eps_abs, double eps_rel, const double2 *y0,
+                         double2 *ynew, double *ratio)
 {
     static const double c[6] = { 0.0, 1.0 / 4, 3.0 / 8, 12.0 / 13, 1.0, 1.0 / 2 };
     static const double a[6][5] = {
@@ -817,7 +1189,7 @@ static int rkf45_attempt(dmd_scatt *h, double t, double hs, double eps_abs, doub
     static const double b4[6] = { 25.0 / 216, 0, 1408.0 / 2565, 2197.0 / 4104, -1.0 / 5, 0 };
     static const double b5[6] = { 16.0 / 135, 0, 6656.0 / 12825, 28561.0 / 56430, -9.0 / 50, 2.0 / 55 };
     const int64_t n = h->nk * (int64_t)h->nbd * h->nbd;
-    double2 *y0 = h->d_ad, *ytmp = h->d_ad + n, *ynew = h->d_ad + 2 * n, *K[6];
+    double2 *ytmp = h->d_ad + n, *K[6];
     for (int j = 0; j < 6; j++) K[j] = h->d_ad + (3 + j) * n;
     int rc;
     if ((rc = set_clock(h, t, hs, 0))) return rc;
@@ -825,7 +1197,27 @@ static int rkf45_attempt(dmd_scatt *h, double t, double hs, double eps_abs, doub
     const dim3 g(nblk(n, 256)), bl(256);
     Ptr6 kp;
     for (int j = 0; j < 6; j++) kp.p[j] = K[j];
-    for (int s = 0; s < 6; s++) {
+    Coef6 cb{}, ce{};
+    for (int j = 0; j < 6; j++) { cb.c[j] = b4[j]; ce.c[j] = b5[j] - b4[j]; }
+    const bool fused = packed_rows(h) && !h->rhs_hook;
+    int nparts = (int)nblk(n, 256);
+    if (fused) {
+        const PackedArgs Q = packed_args(h);
+        nparts = (int)stage_blocks(h);
+        if ((rc = packed_begin(h, y0, c[0]))) return rc;
+        for (int s = 0; s < 6; s++) {
+            const double2 *ys = s ? ytmp : y0;
+            if ((rc = launch_packed_sums(h))) return rc;
+            if (s == 5) {
+                DMD_STAGE(k_stage_rkf_final, A, Q, c[5], ys, y0, hs, cb, ce, kp, eps_abs, eps_rel, ynew, h->d_adpart);
+                break;
+            }
+            Coef6 cf{};
+            for (int j = 0; j <= s; j++) cf.c[j] = a[s + 1][j];
+            DMD_STAGE(k_stage_comb, A, Q, c[s], c[s + 1], ys, y0, hs, s + 1, cf, kp, K[s], ytmp);
+        }
+    }
+    for (int s = 0; s < 6 && !fused; s++) {
         const double2 *ys = y0;
         if (s > 0) {
             Coef6 cf{};
@@ -835,14 +1227,13 @@ static int rkf45_attempt(dmd_scatt *h, double t, double hs, double eps_abs, doub
         }
         if ((rc = full_rhs(h, A, ys, c[s], K[s]))) return rc;
     }
-    Coef6 cb{}, ce{};
-    for (int j = 0; j < 6; j++) { cb.c[j] = b4[j]; ce.c[j] = b5[j] - b4[j]; }
-    hipLaunchKernelGGL(k_rkf_final, g, bl, 0, h->st, n, y0, hs, cb, ce, kp, eps_abs, eps_rel, ynew, h->d_adpart);
-    const int nparts = (int)nblk(n, 256);
-    hipLaunchKernelGGL(k_max_final, dim3(1), dim3(256), 0, h->st, nparts, h->d_adpart, h->d_adpart + nparts);
+    if (!fused)
+        hipLaunchKernelGGL(k_rkf_final, g, bl, 0, h->st, n, y0, hs, cb, ce, kp, eps_abs, eps_rel, ynew, h->d_adpart);
+    // straight into pinned memory: the host waits for the stream, not for a copy
+    hipLaunchKernelGGL(k_max_final, dim3(1), dim3(256), 0, h->st, nparts, h->d_adpart, h->h_ratio);
     DMD_HIP(hipGetLastError());
-    DMD_HIP(hipMemcpyAsync(ratio, h->d_adpart + nparts, 8, hipMemcpyDeviceToHost, h->st));
     DMD_HIP(hipStreamSynchronize(h->st));
+    *ratio = *(volatile double *)h->h_ratio;
     return DMD_OK;
 }
 
@@ -860,6 +1251,7 @@ extern "C" int dmd_scatt_rkf45_apply(dmd_scatt *h, double *t, double t1, double 
     if ((rc = tiles4_prepare(h))) return rc;
     const int64_t n = h->nk * (int64_t)h->nbd * h->nbd;
     if ((rc = to_device(h, h->d_ad, rho, (size_t)n * 16))) return rc;
+    double2 *y0 = h->d_ad, *ynew = h->d_ad + 2 * n;  // change places at every accepted step
     dmd_ode_stats st{};
     double tc = *t, hs = std::min(*h_step, hmax);
     constexpr double S = 0.9, Q = 4.0;
@@ -871,7 +1263,7 @@ extern "C" int dmd_scatt_rkf45_apply(dmd_scatt *h, double *t, double t1, double 
             // an error estimate that never passes would shrink h to nothing: stop instead
             if (!(htry > 0) || tc + htry == tc)
                 return fail(DMD_ERR_STATE, "rkf45: the step size underflowed at t = " + std::to_string(tc));
-            if ((rc = rkf45_attempt(h, tc, htry, eps_abs, eps_rel, &ratio))) return rc;
+            if ((rc = rkf45_attempt(h, tc, htry, eps_abs, eps_rel, y0, ynew, &ratio))) return rc;
             st.rhs_evals += 6;
             if (!(ratio == ratio)) return fail(DMD_ERR_STATE, "rkf45: the error estimate is not finite");
             if (ratio > 1.1 && htry > hmin) {
@@ -883,8 +1275,7 @@ extern "C" int dmd_scatt_rkf45_apply(dmd_scatt *h, double *t, double t1, double 
             }
             break;
         }
-        // accept: y0 <- ynew
-        DMD_HIP(hipMemcpyAsync(h->d_ad, h->d_ad + 2 * n, (size_t)n * 16, hipMemcpyDeviceToDevice, h->st));
+        std::swap(y0, ynew);  // accepted
         tc = final_step ? t1 : tc + htry;
         st.steps++;
         st.last_err_ratio = ratio;
@@ -893,8 +1284,7 @@ extern "C" int dmd_scatt_rkf45_apply(dmd_scatt *h, double *t, double t1, double 
         // a step clamped to land on t1 does not shrink the suggestion
         hs = std::min(hmax, final_step ? std::max(hs, hnext) : hnext);
     }
-    DMD_HIP(hipStreamSynchronize(h->st));
-    if ((rc = from_device(h, rho, h->d_ad, (size_t)n * 16))) return rc;
+    if ((rc = from_device(h, rho, y0, (size_t)n * 16))) return rc;
     DMD_HIP(hipStreamSynchronize(h->st));
     *t = tc;
     *h_step = hs;
@@ -922,7 +1312,6 @@ extern "C" int dmd_scatt_integrate_euler(dmd_scatt *h, double t0, double dt, int
                            h->semiclassical);
         DMD_HIP(hipGetLastError());
     }
-    DMD_HIP(hipStreamSynchronize(h->st));
     if ((rc = from_device(h, rho, y, (size_t)n * 16))) return rc;
     DMD_HIP(hipStreamSynchronize(h->st));
     return DMD_OK;

@@ -142,6 +142,43 @@ __device__ __forceinline__ void herm_of(const double2 *c, double hv[4])
     hv[3] = c[1].y - c[2].y;
 }
 
+// Hermitian element (i, j) of a 4 x 4 matrix from its upper triangle with a
+// real diagonal (how zhemm reads A); one_minus: of 1 - A.
+__device__ __forceinline__ double2 up4(const double2 *A, int i, int j, bool one_minus)
+{
+    double2 v;
+    if (i < j) v = A[i * 4 + j];
+    else if (i > j) v = cconj(A[j * 4 + i]);
+    else v = make_double2(A[i * 5].x, 0.0);
+    if (one_minus) v = make_double2((i == j ? 1.0 : 0.0) - v.x, -v.y);
+    return v;
+}
+
+__device__ __forceinline__ double2 c_elem(const double2 *F, const double2 *rk, const double2 *r1k, int i, int j);
+// X_ij of C = (1-rho) F1 - F2 rho for one row; F as [F1 re/im | F2 re/im];
+// 1-rho from r1k when given (explicit dm1), else formed from rho.
+__device__ __forceinline__ double2 c_elem(const double *F, const double2 *rk, const double2 *r1k, int i, int j)
+{
+    double2 x = make_double2(0, 0);
+#pragma unroll
+    for (int m = 0; m < 4; m++) {
+        const double2 f1 = make_double2(F[2 * (4 * m + j)], F[2 * (4 * m + j) + 1]);
+        cfma(x, r1k ? up4(r1k, i, m, false) : up4(rk, i, m, true), f1);
+    }
+#pragma unroll
+    for (int m = 0; m < 4; m++) {
+        const double2 f2 = make_double2(F[32 + 2 * (4 * i + m)], F[32 + 2 * (4 * i + m) + 1]);
+        cfma(x, make_double2(-f2.x, -f2.y), up4(rk, m, j, false));
+    }
+    return x;
+}
+
+// the same with F as 32 complex [F1 | F2]
+__device__ __forceinline__ double2 c_elem(const double2 *F, const double2 *rk, const double2 *r1k, int i, int j)
+{
+    return c_elem((const double *)F, rk, r1k, i, j);
+}
+
 // Rows [base_row, base_row + 64) of one wave: lane l holds the 4 doubles of
 // row base_row + l (zeros past nk); the wave regroups them so every atomic
 // instruction covers 16 consecutive rows' 32-byte records (4 full lines).
@@ -255,6 +292,9 @@ struct dmd_scatt {
     // adaptive / Euler integrators: 9 states (y0, ytmp, ynew, k1..k6) and the error partials
     double2 *d_ad = nullptr;
     double *d_adpart = nullptr;
+    double *h_ratio = nullptr;           // pinned: the error ratio of an attempt
+    double *d_obs_series = nullptr;      // reports of an integrate_rk4 run
+    int64_t obs_series_cap = 0;
     int64_t ad_cap = 0;
     double2 *d_rhoS = nullptr, *d_rho1S = nullptr, *d_out = nullptr, *d_eq = nullptr;
     // alg_linearize_dPee: the Hermitian row term of the e-e P's change, added
@@ -316,6 +356,18 @@ int set_clock(dmd_scatt *h, double t0, double dt, long long step);
 int launch_rotate(dmd_scatt *h, const double2 *in, const double2 *in1, int nbd, int b0, double a, int semic = 0);
 // contraction + Hermitian epilogue on h->d_rhoS (and h->d_rho1S when dm1) into out (nk x nb^2)
 int launch_contract(dmd_scatt *h, bool dm1, double a, double2 *out);
+// the tile kernels' contraction alone on h->d_rhoS (h->d_x32 for the reduced
+// forms): the packed Hermitian rows in h->d_acc_herm (nb = 2) or h->d_hacc16
+// (nb = 4), for a fused stage kernel that assembles them; only when packed_rows(h)
+int launch_packed_sums(dmd_scatt *h, bool dm1 = false);
+bool packed_rows(const dmd_scatt *h);
+int launch_tiles4_sums(dmd_scatt *h, bool dm1);
+int launch_split_x(dmd_scatt *h);  // h->d_x32 from h->d_rhoS
+// fixed-step RK4 on packed rows (dmd_driver.hip): begin sets the clock to step
+// j of (t0, dt) and prepares the first contraction from y; a step then takes y
+// (rotated) through the stage states Y[0..2] to ynext and advances the clock
+int rk4_packed_begin(dmd_scatt *h, const double2 *y, double t0, double dt, int64_t j);
+int rk4_packed_step(dmd_scatt *h, double dt, const double2 *y, double2 *const Y[3], double2 *acc, double2 *ynext);
 // adds the alg_linearize_dPee row term at the clock time a into out (nk x nb^2)
 int launch_dP_term(dmd_scatt *h, double a, double2 *out);
 // nb = 2: out = prefac/2 x the packed Hermitian rows of h->d_acc_herm, rotated to

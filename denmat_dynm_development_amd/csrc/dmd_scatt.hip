@@ -102,6 +102,43 @@ __global__ void k_rotate_in(int64_t nk, int nbd, int b0, const double2 *__restri
     }
 }
 
+// What one evaluation starts with, in one launch: the clock at time t, the
+// state kept for dmd_scatt_time_eval (keep null: it is there), and the rotation
+// of k_rotate_in (no window).  A copy, a clock kernel and the rotation apart
+// were 5 of the 30 us of a 450-pair evaluation.
+template <int NB>
+__global__ __launch_bounds__(256) void k_eval_in(int64_t nk, const double2 *__restrict__ rho,
+                                                 const double2 *__restrict__ rho1, const double *__restrict__ e,
+                                                 double t, int expt, double2 *__restrict__ rhoS,
+                                                 double2 *__restrict__ rho1S, const double *__restrict__ fsub,
+                                                 double2 *__restrict__ keep, DClock *__restrict__ clk)
+{
+    constexpr int NB2 = NB * NB;
+    const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (idx == 0) {
+        clk->t0 = t;
+        clk->dt = 0.0;
+        clk->step = 0;
+        clk->pad = 0;
+    }
+    if (idx >= nk * NB2) return;
+    const int64_t k = idx / NB2;
+    const int ij = (int)(idx - k * NB2), i = ij / NB, j = ij - i * NB;
+    double2 v = rho[idx], ph = make_double2(1.0, 0.0);
+    if (keep) keep[idx] = v;
+    const bool rot = expt && i != j;
+    if (rot) {
+        ph = ccis(-(e[k * NB + i] - e[k * NB + j]) * t);
+        v = cmul(v, ph);
+    }
+    if (fsub && i == j) v.x -= fsub[k * NB + i];
+    rhoS[idx] = v;
+    if (rho1) {
+        const double2 w = rho1[idx];
+        rho1S[idx] = rot ? cmul(w, ph) : w;
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Row kernel (deterministic): one wavefront per destination row k.
 // Lane roles: element e of a pair's [P1 | P2] (2 NB^4 complex).  For
@@ -860,7 +897,8 @@ dmd_scatt::~dmd_scatt()
     dfree(d_pscale); dfree(d_fsplit); dfree(d_feq); dfree(d_x32); dfree(d_hacc16);
     dfree(d_vrec); dfree(d_bxmax); dfree(d_bqueue); dfree(d_vq); dfree(d_vsd); dfree(d_seg); dfree(d_xb); dfree(d_Fb); dfree(d_rhoSB); dfree(d_bin); dfree(d_bout);
     dfree(d_yB0); dfree(d_yBa); dfree(d_yBb); dfree(d_accB); dfree(d_wB); dfree(d_adj); dfree(d_dotpart);
-    dfree(d_dpos); dfree(d_dk); dfree(d_flin); dfree(d_ad); dfree(d_adpart); dfree(d_phfeq);
+    dfree(d_dpos); dfree(d_dk); dfree(d_flin); dfree(d_ad); dfree(d_adpart); dfree(d_phfeq); dfree(d_obs_series);
+    if (h_ratio) (void)hipHostFree(h_ratio);
     dfree(d_spmask); dfree(d_spgofs); dfree(d_spv);
     for (void *p : extra) dfree(p);
     if (ev0) (void)hipEventDestroy(ev0);
@@ -885,10 +923,17 @@ int from_device(dmd_scatt *h, void *dst, const void *src, size_t bytes)
                            h->st));
     return DMD_OK;
 }
+// by value in a one-thread kernel: a 32-byte copy from pageable memory took
+// 6 us on the stream and blocked the host for as long
+__global__ void k_set_clock(DClock *clk, DClock v)
+{
+    *clk = v;
+}
 int set_clock(dmd_scatt *h, double t0, double dt, long long step)
 {
     h->h_clk.t0 = t0; h->h_clk.dt = dt; h->h_clk.step = step; h->h_clk.pad = 0;
-    DMD_HIP(hipMemcpyAsync(h->d_clk, &h->h_clk, sizeof(DClock), hipMemcpyHostToDevice, h->st));
+    hipLaunchKernelGGL(k_set_clock, dim3(1), dim3(1), 0, h->st, h->d_clk, h->h_clk);
+    DMD_HIP(hipGetLastError());
     return DMD_OK;
 }
 
@@ -913,11 +958,18 @@ static int64_t plan_chunk_len(const std::vector<int64_t> &sizes, int64_t unit, i
                               int64_t lo, int64_t hi)
 {
     constexpr int kCu = 256;
-    int64_t at_lo = 0, best = hi, seen_pieces = 0, seen_longest = 0;
-    for (int64_t n : sizes) at_lo += (n + lo - 1) / lo;
+    int64_t at_lo = 0, total = 0, best = hi, seen_pieces = 0, seen_longest = 0;
+    for (int64_t n : sizes) {
+        at_lo += (n + lo - 1) / lo;
+        total += n;
+    }
     if (at_lo <= kCu) return lo;  // a CU for every shortest piece
-    double best_cost = 1e300;
-    std::vector<int64_t> cu;
+    lo = std::max(lo, std::min(hi, total / (16 * kCu) / unit * unit));  // 16 pieces per CU are fine enough
+    struct Cand {
+        int64_t L, pieces;
+        double bound;  // the least a length can cost: the mean load, or its longest piece
+    };
+    std::vector<Cand> cand;
     for (int64_t L = hi; L >= lo; L = std::min(L - unit, L * 15 / 16 / unit * unit)) {
         int64_t pieces = 0, load = 0, longest = 0;
         for (int64_t n : sizes) {
@@ -930,17 +982,25 @@ static int64_t plan_chunk_len(const std::vector<int64_t> &sizes, int64_t unit, i
         if (pieces == seen_pieces && longest == seen_longest) continue;  // the same pieces as the last length
         seen_pieces = pieces;
         seen_longest = longest;
-        // the mean load is the least the largest can be; with many pieces it is
-        // the estimate, with half a piece at the end
-        double cost = std::max((double)load / kCu, (double)longest) + tail * (double)longest;
-        if (pieces > 16 * kCu) {
-            cost = (double)load / kCu + (0.5 + tail) * (double)longest;
-        } else if (cost < best_cost) {
+        // with many pieces the estimate: the mean load and half a piece at the end
+        cand.push_back({ L, pieces,
+                         pieces > 20 * kCu ? (double)load / kCu + (0.5 + tail) * (double)longest
+                                           : std::max((double)load / kCu, (double)longest) + tail * (double)longest });
+    }
+    std::stable_sort(cand.begin(), cand.end(), [](const Cand &a, const Cand &b) { return a.bound < b.bound; });
+    double best_cost = 1e300;
+    std::vector<int64_t> cu;
+    for (const Cand &c : cand) {
+        if (c.bound >= best_cost) break;
+        double cost = c.bound;
+        if (c.pieces <= 20 * kCu) {
             cu.assign(kCu, 0);  // a heap by load, least first
+            int64_t longest = 0;
             const auto more = std::greater<int64_t>();
             for (int64_t n : sizes) {
                 if (!n) continue;
-                const int64_t m = (n + L - 1) / L, len = ((n + m - 1) / m + unit - 1) / unit * unit;
+                const int64_t m = (n + c.L - 1) / c.L, len = ((n + m - 1) / m + unit - 1) / unit * unit;
+                longest = std::max(longest, len + over);
                 for (int64_t a = 0; a < n; a += len) {
                     std::pop_heap(cu.begin(), cu.end(), more);
                     cu.back() += len + over;
@@ -949,7 +1009,7 @@ static int64_t plan_chunk_len(const std::vector<int64_t> &sizes, int64_t unit, i
             }
             cost = (double)*std::max_element(cu.begin(), cu.end()) + tail * (double)longest;
         }
-        if (cost < best_cost) { best_cost = cost; best = L; }
+        if (cost < best_cost) { best_cost = cost; best = c.L; }
     }
     return best;
 }
@@ -1605,6 +1665,21 @@ int launch_rotate(dmd_scatt *h, const double2 *in, const double2 *in1, int nbd, 
     return DMD_OK;
 }
 
+static int launch_eval_in(dmd_scatt *h, double t, const double2 *in, const double2 *in1, double2 *keep)
+{
+    const double *fs = h->linear ? h->d_flin : nullptr;
+    const dim3 g(nblk(h->nk * h->nb2, 256)), b(256);
+    h->h_clk = DClock{ t, 0.0, 0, 0 };
+    switch (h->nb) {
+    case 1: hipLaunchKernelGGL(k_eval_in<1>, g, b, 0, h->st, h->nk, in, in1, h->d_e, t, h->expt, h->d_rhoS, h->d_rho1S, fs, keep, h->d_clk); break;
+    case 2: hipLaunchKernelGGL(k_eval_in<2>, g, b, 0, h->st, h->nk, in, in1, h->d_e, t, h->expt, h->d_rhoS, h->d_rho1S, fs, keep, h->d_clk); break;
+    case 3: hipLaunchKernelGGL(k_eval_in<3>, g, b, 0, h->st, h->nk, in, in1, h->d_e, t, h->expt, h->d_rhoS, h->d_rho1S, fs, keep, h->d_clk); break;
+    case 4: hipLaunchKernelGGL(k_eval_in<4>, g, b, 0, h->st, h->nk, in, in1, h->d_e, t, h->expt, h->d_rhoS, h->d_rho1S, fs, keep, h->d_clk); break;
+    }
+    DMD_HIP(hipGetLastError());
+    return DMD_OK;
+}
+
 template <int NB>
 static void launch_rows_nb(dmd_scatt *h, bool dm1, double a, double2 *out)
 {
@@ -1653,9 +1728,9 @@ int launch_raw_rows(dmd_scatt *h, const double2 *X, const double2 *Y)
     return DMD_OK;
 }
 
-static void launch_tiles(dmd_scatt *h, bool dm1, double a, double2 *out)
+// the contraction alone: packed Hermitian rows added into d_acc_herm
+static void launch_tiles_sums(dmd_scatt *h, bool dm1)
 {
-    const double2 *eq = h->has_eq ? h->d_eq : nullptr;
     if (h->ngroups > 0) {
         if (h->linear)
             hipLaunchKernelGGL((k_tiles_soa<false, true>), dim3((unsigned)h->ngroups), dim3(256), 0, h->st, h->nk, h->d_P,
@@ -1675,6 +1750,12 @@ static void launch_tiles(dmd_scatt *h, bool dm1, double a, double2 *out)
             hipLaunchKernelGGL((k_tiles_soa<false, false>), dim3((unsigned)h->ngroups), dim3(256), 0, h->st, h->nk, h->d_P,
                                h->d_pk, h->d_cbeg, h->d_clen, h->d_cij, h->d_gbeg, h->d_rhoS, h->d_rho1S, h->d_acc_herm);
     }
+}
+
+static void launch_tiles(dmd_scatt *h, bool dm1, double a, double2 *out)
+{
+    const double2 *eq = h->has_eq ? h->d_eq : nullptr;
+    launch_tiles_sums(h, dm1);
     hipLaunchKernelGGL(k_assemble_h, dim3(nblk(h->nk, 256)), dim3(256), 0, h->st, h->nk, h->d_acc_herm, h->d_e,
                        h->d_clk, a, h->expt, h->schrodinger, h->prefac, eq, out);
 }
@@ -1688,6 +1769,20 @@ int contract_kind(const dmd_scatt *h)
     if (h->kernel == DMD_KERNEL_ROWS || h->nb > 2) return DMD_KERNEL_ROWS;
     if (h->kernel == DMD_KERNEL_SINGLE_READ) return DMD_KERNEL_SINGLE_READ;
     return h->nb == 2 && h->tile_R ? DMD_KERNEL_TILES : DMD_KERNEL_SINGLE_READ;
+}
+
+bool packed_rows(const dmd_scatt *h)
+{
+    return contract_kind(h) == DMD_KERNEL_TILES && (h->linear || !h->has_dP);
+}
+
+int launch_packed_sums(dmd_scatt *h, bool dm1)
+{
+    if (!packed_rows(h)) return fail(DMD_ERR_STATE, "packed row sums are a tile-kernel form");
+    if (h->nb == 4) return launch_tiles4_sums(h, dm1);
+    launch_tiles_sums(h, dm1);
+    DMD_HIP(hipGetLastError());
+    return DMD_OK;
 }
 
 // the contraction + epilogue on the current rhoS (and rho1S when dm1)
@@ -1752,15 +1847,17 @@ static int eval_core(dmd_scatt *h, double t, const double *rho, const double *rh
     int rc;
     const double2 *in = (const double2 *)rho, *in1 = (const double2 *)rho1;
     // the state always lands in d_in (dmd_scatt_time_eval replays it)
-    if ((rc = to_device(h, h->d_in, rho, bytes))) return rc;
-    in = h->d_in;
+    const bool dev = is_device_ptr(rho);
+    if (!dev) {
+        if ((rc = to_device(h, h->d_in, rho, bytes))) return rc;
+        in = h->d_in;
+    }
     if (rho1 && !is_device_ptr(rho1)) {
         if ((rc = to_device(h, h->d_in1, rho1, bytes))) return rc;
         in1 = h->d_in1;
     }
     if ((rc = tiles4_prepare(h))) return rc;
-    if ((rc = set_clock(h, t, 0.0, 0))) return rc;
-    if ((rc = launch_rotate(h, in, in1, h->nb, 0, 0.0))) return rc;
+    if ((rc = launch_eval_in(h, t, in, in1, dev ? h->d_in : nullptr))) return rc;
     double2 *out = is_device_ptr(ddmdt) ? (double2 *)ddmdt : h->d_out;
     if (timed) DMD_HIP(hipEventRecord(h->ev0, h->st));
     if ((rc = launch_contract(h, rho1 != nullptr, 0.0, out))) return rc;

@@ -158,43 +158,6 @@ template <typename V> struct Loader<bf16c, V> {
     }
 };
 
-// Hermitian element (i, j) of a 4 x 4 matrix from its upper triangle with a
-// real diagonal (how zhemm reads A); one_minus: of 1 - A.
-__device__ __forceinline__ double2 up4(const double2 *A, int i, int j, bool one_minus)
-{
-    double2 v;
-    if (i < j) v = A[i * 4 + j];
-    else if (i > j) v = cconj(A[j * 4 + i]);
-    else v = make_double2(A[i * 5].x, 0.0);
-    if (one_minus) v = make_double2((i == j ? 1.0 : 0.0) - v.x, -v.y);
-    return v;
-}
-
-__device__ __forceinline__ double2 c_elem(const double2 *F, const double2 *rk, const double2 *r1k, int i, int j);
-// X_ij of C = (1-rho) F1 - F2 rho for one row; F as [F1 re/im | F2 re/im];
-// 1-rho from r1k when given (explicit dm1), else formed from rho.
-__device__ __forceinline__ double2 c_elem(const double *F, const double2 *rk, const double2 *r1k, int i, int j)
-{
-    double2 x = make_double2(0, 0);
-#pragma unroll
-    for (int m = 0; m < 4; m++) {
-        const double2 f1 = make_double2(F[2 * (4 * m + j)], F[2 * (4 * m + j) + 1]);
-        cfma(x, r1k ? up4(r1k, i, m, false) : up4(rk, i, m, true), f1);
-    }
-#pragma unroll
-    for (int m = 0; m < 4; m++) {
-        const double2 f2 = make_double2(F[32 + 2 * (4 * i + m)], F[32 + 2 * (4 * i + m) + 1]);
-        cfma(x, make_double2(-f2.x, -f2.y), up4(rk, m, j, false));
-    }
-    return x;
-}
-
-// the same with F as 32 complex [F1 | F2]
-__device__ __forceinline__ double2 c_elem(const double2 *F, const double2 *rk, const double2 *r1k, int i, int j)
-{
-    return c_elem((const double *)F, rk, r1k, i, j);
-}
-
 // Packed Hermitian increment of element l = 4i + j: H_ii (i == j), Re H_ij
 // (i < j), Im H_ji (i > j), from X = C of the row.
 __device__ __forceinline__ double herm_pack(double2 xij, double2 xji, int i, int j)
@@ -444,6 +407,12 @@ __global__ __launch_bounds__(256) void k_assemble_h4(int64_t nk, double *__restr
     const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t k = idx >> 4;
     const int l = (int)(idx & 15), i = l >> 2, j = l & 3;
+    // the block's rows of rho (an indexed private copy would sit in scratch)
+    __shared__ double2 rows[256];
+    if (feq) {
+        rows[threadIdx.x] = k < nk ? rhoS[idx] : make_double2(0, 0);
+        __syncthreads();
+    }
     double2 d = make_double2(0, 0);
     if (k < nk) {
         const double *h = hacc + k * 16;
@@ -451,9 +420,7 @@ __global__ __launch_bounds__(256) void k_assemble_h4(int64_t nk, double *__restr
         else if (i < j) d = make_double2(h[4 * i + j], h[4 * j + i]);
         else d = make_double2(h[4 * j + i], -h[4 * i + j]);
         if (feq) {
-            double2 rk[16];
-#pragma unroll
-            for (int q = 0; q < 16; q++) rk[q] = rhoS[k * 16 + q];
+            const double2 *rk = rows + (threadIdx.x & ~15);
             const double *F = feq + k * 64;
             const double2 xij = c_elem(F, rk, nullptr, i, j), xji = c_elem(F, rk, nullptr, j, i);
             d = cadd(d, cadd(xij, cconj(xji)));
@@ -754,22 +721,41 @@ int tiles4_prepare(dmd_scatt *h)
     return DMD_OK;
 }
 
+int launch_split_x(dmd_scatt *h)
+{
+    hipLaunchKernelGGL(k_split_x, dim3(nblk(h->nk * 16, 256)), dim3(256), 0, h->st, h->nk, h->d_rhoS, h->d_fsplit,
+                       h->d_x32);
+    DMD_HIP(hipGetLastError());
+    return DMD_OK;
+}
+
+// the contraction alone (rows added into d_hacc16), on the current rhoS (and
+// rho1S when dm1) or, for the reduced forms, x32
+int launch_tiles4_sums(dmd_scatt *h, bool dm1)
+{
+    if (h->linear) {
+        launch_k4<double2, double, false, false, false, true>(h, h->d_rhoS, nullptr, h->d_hacc16);
+    } else if (h->precision == DMD_PREC_FP64) {
+        if (dm1) launch_k4<double2, double, false, false, true>(h, h->d_rhoS, h->d_rho1S, h->d_hacc16);
+        else launch_k4<double2, double, false, false>(h, h->d_rhoS, nullptr, h->d_hacc16);
+    } else if (h->precision == DMD_PREC_C64) {
+        launch_k4<float2, float, false, true>(h, h->d_x32, nullptr, h->d_hacc16);
+    } else {
+        launch_k4<bf16c, float, false, true>(h, h->d_x32, nullptr, h->d_hacc16);
+    }
+    DMD_HIP(hipGetLastError());
+    return DMD_OK;
+}
+
 // contraction + epilogue for nb = 4 on the current rhoS (and rho1S when dm1;
 // the reduced forms always form 1 - rho from rho) into out
 int launch_tiles4(dmd_scatt *h, bool dm1, double a, double2 *out)
 {
     const double2 *eq = h->has_eq ? h->d_eq : nullptr;
     const int64_t n16 = h->nk * 16;
-    if (h->linear) {
-        launch_k4<double2, double, false, false, false, true>(h, h->d_rhoS, nullptr, h->d_hacc16);
-    } else if (h->precision == DMD_PREC_FP64) {
-        if (dm1) launch_k4<double2, double, false, false, true>(h, h->d_rhoS, h->d_rho1S, h->d_hacc16);
-        else launch_k4<double2, double, false, false>(h, h->d_rhoS, nullptr, h->d_hacc16);
-    } else {
-        hipLaunchKernelGGL(k_split_x, dim3(nblk(n16, 256)), dim3(256), 0, h->st, h->nk, h->d_rhoS, h->d_fsplit, h->d_x32);
-        if (h->precision == DMD_PREC_C64) launch_k4<float2, float, false, true>(h, h->d_x32, nullptr, h->d_hacc16);
-        else launch_k4<bf16c, float, false, true>(h, h->d_x32, nullptr, h->d_hacc16);
-    }
+    int rc;
+    if (h->precision != DMD_PREC_FP64 && !h->linear && (rc = launch_split_x(h))) return rc;
+    if ((rc = launch_tiles4_sums(h, dm1))) return rc;
     hipLaunchKernelGGL(k_assemble_h4, dim3(nblk(n16, 256)), dim3(256), 0, h->st, h->nk, h->d_hacc16,
                        h->precision == DMD_PREC_FP64 ? nullptr : h->d_feq, h->d_rhoS, h->d_e, h->d_clk, a, h->expt,
                        h->schrodinger, h->prefac, eq, out);
