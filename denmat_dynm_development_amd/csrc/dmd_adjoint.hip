@@ -435,6 +435,116 @@ __global__ __launch_bounds__(256) void k_tiles_vjp(int64_t nk, const double2 *__
     }
 }
 
+// ---------------------------------------------------------------------------
+// The reverse sweep's element-wise work between two VJP passes, one thread per
+// k (nb = 2), in one launch each (six or seven of about 4 us apart).  Stage
+// times come by value.
+// ---------------------------------------------------------------------------
+struct AdjArgs {
+    int64_t nk;
+    double *hacc;       // packed rows of the VJP pass (cleared here)
+    double scale;       // prefac / 4
+    const double *e;
+    int expt;
+};
+// g = Herm(prefac/2 s) e^{i w t} of the pass's packed rows
+__device__ __forceinline__ void adj_take(const AdjArgs &A, int64_t k, double t, double2 g[4])
+{
+    double *h = A.hacc + k * 4;
+    const double h0 = h[0], h1 = h[1], hr = h[2], hi = h[3];
+    h[0] = 0.0; h[1] = 0.0; h[2] = 0.0; h[3] = 0.0;
+    g[0] = make_double2(h0 * A.scale, 0.0);
+    g[3] = make_double2(h1 * A.scale, 0.0);
+    g[1] = make_double2(hr * A.scale, hi * A.scale);
+    if (A.expt) g[1] = cmul(g[1], ccis((A.e[2 * k] - A.e[2 * k + 1]) * t));
+    g[2] = cconj(g[1]);
+}
+// rho_S = y e^{-i w t}, u_S = v_S + v_S^+ with v_S = v e^{-i w t}
+__device__ __forceinline__ void adj_stage_in(const AdjArgs &A, int64_t k, double t, const double2 *y,
+                                             const double2 v[4], double2 *rS, double2 *uS)
+{
+    double2 ph = make_double2(1.0, 0.0);
+    if (A.expt) ph = ccis(-(A.e[2 * k] - A.e[2 * k + 1]) * t);
+    const double2 *yk = y + k * 4;
+    double2 *r = rS + k * 4, *u = uS + k * 4;
+    r[0] = yk[0];
+    r[1] = cmul(yk[1], ph);
+    r[2] = cmul(yk[2], cconj(ph));
+    r[3] = yk[3];
+    const double2 v1 = cmul(v[1], ph), v2 = cmul(v[2], cconj(ph));
+    u[0] = make_double2(2.0 * v[0].x, 0.0);
+    u[1] = cadd(v1, cconj(v2));
+    u[2] = cadd(v2, cconj(v1));
+    u[3] = make_double2(2.0 * v[3].x, 0.0);
+}
+// after the pass of stage s = 3, 2, 1: ynew += g and the operands of stage s - 1,
+// whose slope's cotangent is w z + back g
+__global__ __launch_bounds__(64) void k_adj_stage(AdjArgs A, double t, double2 *__restrict__ ynew,
+                                                  const double2 *__restrict__ z, double w, double back,
+                                                  const double2 *__restrict__ yprev, double tprev,
+                                                  double2 *__restrict__ rS, double2 *__restrict__ uS)
+{
+    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= A.nk) return;
+    double2 g[4], v[4];
+    adj_take(A, k, t, g);
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const double2 zq = z[k * 4 + q];
+        ynew[k * 4 + q] = cadd(ynew[k * 4 + q], g[q]);
+        v[q] = make_double2(w * zq.x + back * g[q].x, w * zq.y + back * g[q].y);
+    }
+    adj_stage_in(A, k, tprev, yprev, v, rS, uS);
+}
+// The end of a step (take: after the pass of its stage 0 at time t) and the
+// start of the one before it (y3: that step's stage-3 state, at time t3): ybar =
+// ynew + g (take; else ybar as it is), plus the observable's cotangent w_obs
+// conj(s_t) at t, then z = ynew = Herm(ybar) and stage 3's operands from w3 z.
+__global__ __launch_bounds__(64) void k_adj_step(AdjArgs A, int take, double t, double2 *__restrict__ ybar,
+                                                 double2 *__restrict__ ynew, double w_obs, const double2 *__restrict__ s,
+                                                 const double *__restrict__ edm, int i0, int i1,
+                                                 double2 *__restrict__ z, const double2 *__restrict__ y3, double t3,
+                                                 double w3, double2 *__restrict__ rS, double2 *__restrict__ uS)
+{
+    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= A.nk) return;
+    double2 y[4];
+    if (take) {
+        adj_take(A, k, t, y);
+#pragma unroll
+        for (int q = 0; q < 4; q++) y[q] = cadd(ynew[k * 4 + q], y[q]);
+    } else {
+#pragma unroll
+        for (int q = 0; q < 4; q++) y[q] = ybar[k * 4 + q];
+    }
+    if (w_obs != 0.0) {
+        const double2 ph = ccis((edm[2 * k] - edm[2 * k + 1]) * t);
+#pragma unroll
+        for (int q = 0; q < 4; q++) {  // y[b][i] += w conj(s_t[i][b])
+            const int b = q >> 1, i = q & 1;
+            if (i < i0 || i >= i1) continue;
+            double2 sk = s[k * 4 + i * 2 + b];
+            if (i != b) sk = cmul(sk, i == 0 ? ph : cconj(ph));
+            y[q] = make_double2(y[q].x + w_obs * sk.x, y[q].y - w_obs * sk.y);
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) ybar[k * 4 + q] = y[q];
+    if (!y3) return;
+    double2 h[4];
+    h[0] = make_double2(y[0].x, 0.0);
+    h[3] = make_double2(y[3].x, 0.0);
+    h[1] = make_double2(0.5 * (y[1].x + y[2].x), 0.5 * (y[1].y - y[2].y));
+    h[2] = cconj(h[1]);
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        z[k * 4 + q] = h[q];
+        ynew[k * 4 + q] = h[q];
+        h[q] = make_double2(w3 * h[q].x, w3 * h[q].y);
+    }
+    adj_stage_in(A, k, t3, y3, h, rS, uS);
+}
+
 // The parameter cotangents through P (nb = 2): the scattering term is linear
 // in P, and Re <v, f_P(rho)> = prefac/2 Re sum_pairs sum_mn (P1[m,n] G1[m,n] +
 // P2[m,n] G2[m,n]) with, in the Schroedinger picture (vec index m = (i1 i2),
@@ -448,7 +558,7 @@ __global__ __launch_bounds__(256) void k_tiles_vjp(int64_t nk, const double2 *__
 __global__ __launch_bounds__(256) void k_adj_G(int64_t nslots, const int32_t *__restrict__ k1,
                                                const int32_t *__restrict__ k2, int nst, int64_t stride,
                                                const double2 *__restrict__ rS, const double2 *__restrict__ uS,
-                                               double2 *__restrict__ Gc)
+                                               int first, double2 *__restrict__ Gc)
 {
     constexpr int NB2 = 4, NB4 = 16, EP = 32;
     // Workgroups run on XCD w % 8 (the hardware's round-robin), so XCD x
@@ -460,13 +570,19 @@ __global__ __launch_bounds__(256) void k_adj_G(int64_t nslots, const int32_t *__
     const int64_t s = bid * blockDim.x + threadIdx.x;
     if (s >= nslots) return;
     const int32_t ka = k1[s];
-    if (ka < 0) return;  // padding slot
+    double2 *g = Gc + (s >> 3) * (8 * EP) + (s & 7);
+    if (ka < 0) {  // padding slot
+        for (int el = 0; first && el < 2 * NB4; el++) g[el * 8] = make_double2(0.0, 0.0);
+        return;
+    }
     const int64_t a = ka, bk = k2[s];
     const bool rev = a < bk;
-    double2 *g = Gc + (s >> 3) * (8 * EP) + (s & 7);
     double2 g1[NB4], g2[NB4];
 #pragma unroll
-    for (int el = 0; el < NB4; el++) { g1[el] = g[el * 8]; g2[el] = g[(NB4 + el) * 8]; }
+    for (int el = 0; el < NB4; el++) {  // the first fold starts the sums
+        g1[el] = first ? make_double2(0.0, 0.0) : g[el * 8];
+        g2[el] = first ? make_double2(0.0, 0.0) : g[(NB4 + el) * 8];
+    }
     for (int st = 0; st < nst; st++) {
         double2 rk[NB2], uk[NB2], rp[NB2], up[NB2], xk[NB2], yk[NB2], xp[NB2], yp[NB2];
 #pragma unroll
@@ -496,13 +612,56 @@ __global__ __launch_bounds__(256) void k_adj_G(int64_t nslots, const int32_t *__
     for (int el = 0; el < NB4; el++) { g[el * 8] = g1[el]; g[(NB4 + el) * 8] = g2[el]; }
 }
 
-// y[0] += c x[0]; x[0] = 0
-__global__ void k_take_scaled(double *__restrict__ x, double c, double *__restrict__ y)
+// dtheta_c = scale_c Re <Gc, P_c> of up to kDots components in one read of Gc
+constexpr int kDots = 8;
+struct DotArgs {
+    const double2 *p[kDots];
+    double scale[kDots];
+    int n;
+};
+__global__ __launch_bounds__(256) void k_dots_partial(int64_t n, const double2 *__restrict__ g, DotArgs D,
+                                                      double *__restrict__ part)
 {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        y[0] += c * x[0];
-        x[0] = 0.0;
+    __shared__ double red[256];
+    double s[kDots];
+#pragma unroll
+    for (int c = 0; c < kDots; c++) s[c] = 0.0;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+        const double2 v = ld_stream(g + i);
+#pragma unroll
+        for (int c = 0; c < kDots; c++)
+            if (c < D.n) {
+                const double2 p = ld_stream(D.p[c] + i);
+                s[c] += v.x * p.x + v.y * p.y;
+            }
     }
+#pragma unroll
+    for (int c = 0; c < kDots; c++) {
+        if (c >= D.n) break;
+        __syncthreads();
+        red[threadIdx.x] = s[c];
+        __syncthreads();
+        for (int w = 128; w > 0; w >>= 1) {
+            if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
+            __syncthreads();
+        }
+        if (threadIdx.x == 0) part[(int64_t)c * gridDim.x + blockIdx.x] = red[0];
+    }
+}
+__global__ __launch_bounds__(256) void k_dots_final(int nparts, const double *__restrict__ part, DotArgs D,
+                                                    double *__restrict__ out)
+{
+    __shared__ double red[256];
+    const int c = blockIdx.x;
+    double s = 0;
+    for (int i = threadIdx.x; i < nparts; i += 256) s += part[(int64_t)c * nparts + i];
+    red[threadIdx.x] = s;
+    __syncthreads();
+    for (int w = 128; w > 0; w >>= 1) {
+        if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) out[c] = D.scale[c] * red[0];
 }
 // y = 0 (fresh allocations may hold any bit pattern, NaN included)
 __global__ void k_zero2(int64_t n, double2 *__restrict__ y)
@@ -565,6 +724,16 @@ static int launch_vjp_nb(dmd_scatt *h, const double2 *y, const double2 *v, doubl
     return DMD_OK;
 }
 
+// the tile VJP's pass alone on prepared operands: packed rows into d_acc_herm
+static int launch_vjp_pass(dmd_scatt *h, const double2 *rS, const double2 *uS)
+{
+    if (h->ngroups > 0)
+        hipLaunchKernelGGL(k_tiles_vjp, dim3((unsigned)h->ngroups), dim3(256), 0, h->st, h->nk, h->d_P, h->d_pk,
+                           h->d_cbeg, h->d_clen, h->d_cij, h->d_gbeg, rS, uS, h->d_acc_herm);
+    DMD_HIP(hipGetLastError());
+    return DMD_OK;
+}
+
 // One-pass tile VJP at stage a of the clock: rho_S, u_S into rS, uS (kept
 // for the parameter cotangents), then the pass and the epilogue into g.
 static int launch_vjp_tiles(dmd_scatt *h, const double2 *y, const double2 *v, double a, double2 *rS, double2 *uS,
@@ -572,10 +741,8 @@ static int launch_vjp_tiles(dmd_scatt *h, const double2 *y, const double2 *v, do
 {
     hipLaunchKernelGGL(k_vjp_stage_in<2>, dim3(nblk(h->nk, 256)), dim3(256), 0, h->st, h->nk, y, v, h->d_e, h->d_clk, a,
                        h->expt, rS, uS);
-    if (h->ngroups > 0)
-        hipLaunchKernelGGL(k_tiles_vjp, dim3((unsigned)h->ngroups), dim3(256), 0, h->st, h->nk, h->d_P, h->d_pk,
-                           h->d_cbeg, h->d_clen, h->d_cij, h->d_gbeg, rS, uS, h->d_acc_herm);
-    DMD_HIP(hipGetLastError());
+    const int rc = launch_vjp_pass(h, rS, uS);
+    if (rc) return rc;
     return launch_assemble_herm(h, a, 0.5 * h->prefac, g);
 }
 
@@ -731,8 +898,8 @@ extern "C" int dmd_scatt_adjoint_rk4(dmd_scatt *h, double t0, double dt, int64_t
     const int64_t gwords = tiles && ncomp > 0 ? h->nslots * 2 * h->nb4 : 0;
     if (gwords) {
         if ((rc = alloc(&Gc, (size_t)gwords, "parameter cotangent sums"))) return rc;
-        hipLaunchKernelGGL(k_zero2, dim3(nblk(gwords, 256)), dim3(256), 0, h->st, gwords, Gc);
     }
+    bool first_fold = true;
     // the parameter fold runs once per kGroup steps over their 4 kGroup stages
     constexpr int kGroup = 4;
     if (tiles && ((rc = alloc(&rS, 4 * kGroup * n, "stage rho_S")) || (rc = alloc(&uS, 4 * kGroup * n, "stage u_S"))))
@@ -741,7 +908,8 @@ extern "C" int dmd_scatt_adjoint_rk4(dmd_scatt *h, double t0, double dt, int64_t
     auto fold_G = [&]() -> int {
         if (gwords && pending > 0 && h->nslots > 0)
             hipLaunchKernelGGL(k_adj_G, dim3((nblk(h->nslots, 256) + 7) / 8 * 8), dim3(256), 0, h->st, h->nslots,
-                               h->d_k1, h->d_k2, pending, (int64_t)n, rS, uS, Gc);
+                               h->d_k1, h->d_k2, pending, (int64_t)n, rS, uS, first_fold ? 1 : 0, Gc);
+        if (pending > 0) first_fold = false;
         pending = 0;
         DMD_HIP(hipGetLastError());
         return DMD_OK;
@@ -751,7 +919,7 @@ extern "C" int dmd_scatt_adjoint_rk4(dmd_scatt *h, double t0, double dt, int64_t
         mem.push_back(d_dth);
         DMD_HIP(hipMemsetAsync(d_dth, 0, ncomp * sizeof(double), h->st));
     }
-    if (!h->d_dotpart && (rc = dalloc_t(&h->d_dotpart, 1024, "dot partials"))) return rc;
+    if (!h->d_dotpart && (rc = dalloc_t(&h->d_dotpart, 1024 * kDots, "dot partials"))) return rc;
     std::vector<double> hobs(nobs, 0.0);
     if (nobs) {
         if (is_device_ptr(dL_dobs)) DMD_HIP(hipMemcpy(hobs.data(), dL_dobs, nobs * 8, hipMemcpyDeviceToHost));
@@ -791,11 +959,13 @@ extern "C" int dmd_scatt_adjoint_rk4(dmd_scatt *h, double t0, double dt, int64_t
     auto run_segment = [&](int64_t c) -> int {
         const int64_t j0 = c * C, j1 = std::min<int64_t>(n_steps, (c + 1) * C);
         DMD_HIP(hipMemcpyAsync(stage(0, 0), cp + c * n, bytes, hipMemcpyDeviceToDevice, h->st));
+        int r;
+        if (tiles && (r = rk4_packed_begin(h, stage(0, 0), t0, dt, j0))) return r;
         for (int64_t j = j0; j < j1; j++) {
             double2 *const Y[3] = { stage(j - j0, 1), stage(j - j0, 2), stage(j - j0, 3) };
             double2 *next = j + 1 < j1 ? stage(j + 1 - j0, 0) : cp + (c + 1) * n;
-            int r;
-            if ((r = step(j, stage(j - j0, 0), Y, next))) return r;
+            if ((r = tiles ? rk4_packed_step(h, dt, stage(j - j0, 0), Y, Ks, next) : step(j, stage(j - j0, 0), Y, next)))
+                return r;
         }
         return DMD_OK;
     };
@@ -809,12 +979,13 @@ extern "C" int dmd_scatt_adjoint_rk4(dmd_scatt *h, double t0, double dt, int64_t
         }
         // states ping-pong between tmp and tmp + n; stage states are scratch
         DMD_HIP(hipMemcpyAsync(tmp, cp + c * n, bytes, hipMemcpyDeviceToDevice, h->st));
+        if (tiles && (rc = rk4_packed_begin(h, tmp, t0, dt, c * C))) return rc;
         for (int64_t j = c * C; j < (c + 1) * C; j++) {
             double2 *const Y[3] = { stage(0, 1), stage(0, 2), stage(0, 3) };
             const int64_t q = j - c * C;
             const double2 *y = tmp + (q % 2 ? n : 0);
             double2 *next = j + 1 < (c + 1) * C ? tmp + (q % 2 ? 0 : n) : cp + (c + 1) * n;
-            if ((rc = step(j, y, Y, next))) return rc;
+            if ((rc = tiles ? rk4_packed_step(h, dt, y, Y, Ks, next) : step(j, y, Y, next))) return rc;
         }
     }
     // reverse sweep
@@ -830,12 +1001,42 @@ extern "C" int dmd_scatt_adjoint_rk4(dmd_scatt *h, double t0, double dt, int64_t
         DMD_HIP(hipGetLastError());
         return DMD_OK;
     };
-    if ((rc = add_obs(n_steps))) return rc;
+    if (!tiles && (rc = add_obs(n_steps))) return rc;
+    // tiles: the element-wise work of the sweep in one launch per stage
+    const AdjArgs adj{ nk, h->d_acc_herm, 0.25 * h->prefac, h->d_e, h->expt };
+    const dim3 gk(nblk(nk, 64)), b64(64);
+    auto t_at = [&](int64_t j, double a) { return (t0 + (double)j * dt) + a * dt; };  // as the device clock
+    auto obs_w = [&](int64_t j) { return obs && j % report_every == 0 ? hobs[j / report_every] * h->obs_prefac : 0.0; };
     const double ws[4] = { dt / 6.0, dt / 3.0, dt / 3.0, dt / 6.0 };
     const double back[4] = { 0.0, 0.5 * dt, 0.5 * dt, dt };  // Y_s = y + back_s K_{s-1}
     for (int64_t c = ncp - 1; c >= 0; c--) {
         const int64_t j0 = c * C, j1 = std::min<int64_t>(n_steps, (c + 1) * C);
         if (c + 1 < ncp && (rc = run_segment(c))) return rc;
+        if (tiles) {
+            double2 *zb = kbar;
+            auto slot = [&](double2 *base, int s) { return base + (size_t)(pending + s) * n; };
+            hipLaunchKernelGGL(k_adj_step, gk, b64, 0, h->st, adj, 0, t_at(j1, 0.0), ybar, ynew,
+                               c + 1 == ncp ? obs_w(j1) : 0.0, h->d_s, h->d_edm, h->obs_i0, h->obs_i1, zb,
+                               stage(j1 - 1 - j0, 3), t_at(j1 - 1, a_s[3]), ws[3], slot(rS, 3), slot(uS, 3));
+            for (int64_t j = j1 - 1; j >= j0; j--) {
+                for (int s = 3; s > 0; s--) {
+                    if ((rc = launch_vjp_pass(h, slot(rS, s), slot(uS, s)))) return rc;
+                    hipLaunchKernelGGL(k_adj_stage, gk, b64, 0, h->st, adj, t_at(j, a_s[s]), ynew, zb, ws[s - 1],
+                                       back[s], stage(j - j0, s - 1), t_at(j, a_s[s - 1]), slot(rS, s - 1),
+                                       slot(uS, s - 1));
+                }
+                if ((rc = launch_vjp_pass(h, slot(rS, 0), slot(uS, 0)))) return rc;
+                pending += 4;
+                if (pending == 4 * kGroup && (rc = fold_G())) return rc;
+                const bool more = j > j0;
+                hipLaunchKernelGGL(k_adj_step, gk, b64, 0, h->st, adj, 1, t_at(j, 0.0), ybar, ynew, obs_w(j), h->d_s,
+                                   h->d_edm, h->obs_i0, h->obs_i1, zb,
+                                   more ? (const double2 *)stage(j - 1 - j0, 3) : nullptr, t_at(j - 1, a_s[3]), ws[3],
+                                   slot(rS, 3), slot(uS, 3));
+                DMD_HIP(hipGetLastError());
+            }
+            continue;
+        }
         for (int64_t j = j1 - 1; j >= j0; j--) {
             // zbar = Herm(ybar); Kbar_s = w_s zbar
             double2 *Kb[4] = { kbar, kbar + n, kbar + 2 * n, kbar + 3 * n };
@@ -844,28 +1045,19 @@ extern "C" int dmd_scatt_adjoint_rk4(dmd_scatt *h, double t0, double dt, int64_t
             if ((rc = set_clock(h, t0, dt, j))) return rc;
             for (int s = 3; s >= 0; s--) {
                 const double2 *Y = stage(j - j0, s);
-                if (!tiles) {
-                    // parameter cotangents Re <Kbar_s, f_c(Y_s)>: each component
-                    // evaluates on its own stream, the dot runs on the handle's
-                    for (int cc = 0; cc < ncomp; cc++) {
-                        DMD_HIP(hipStreamSynchronize(h->st));
-                        if ((rc = rhs(comps[cc], j, a_s[s], Y, tmp))) return rc;
-                        DMD_HIP(hipStreamSynchronize(comps[cc]->st));
-                        if ((rc = launch_dot(h, (int64_t)n, Kb[s], tmp, d_dth + cc))) return rc;
-                    }
-                    if ((rc = set_clock(h, t0, dt, j))) return rc;
-                    if ((rc = launch_vjp(h, Y, Kb[s], a_s[s], tmp))) return rc;
-                } else {
-                    const size_t slot = (size_t)(pending + s) * n;
-                    if ((rc = launch_vjp_tiles(h, Y, Kb[s], a_s[s], rS + slot, uS + slot, tmp))) return rc;
+                // parameter cotangents Re <Kbar_s, f_c(Y_s)>: each component
+                // evaluates on its own stream, the dot runs on the handle's
+                for (int cc = 0; cc < ncomp; cc++) {
+                    DMD_HIP(hipStreamSynchronize(h->st));
+                    if ((rc = rhs(comps[cc], j, a_s[s], Y, tmp))) return rc;
+                    DMD_HIP(hipStreamSynchronize(comps[cc]->st));
+                    if ((rc = launch_dot(h, (int64_t)n, Kb[s], tmp, d_dth + cc))) return rc;
                 }
+                if ((rc = set_clock(h, t0, dt, j))) return rc;
+                if ((rc = launch_vjp(h, Y, Kb[s], a_s[s], tmp))) return rc;
                 // Ybar_s = J_s^T Kbar_s
                 hipLaunchKernelGGL(k_acc, gn, b256, 0, h->st, (int64_t)n, 1.0, tmp, ynew);
                 if (s > 0) hipLaunchKernelGGL(k_acc, gn, b256, 0, h->st, (int64_t)n, back[s], tmp, Kb[s - 1]);
-            }
-            if (tiles) {
-                pending += 4;
-                if (pending == 4 * kGroup && (rc = fold_G())) return rc;
             }
             DMD_HIP(hipGetLastError());
             DMD_HIP(hipMemcpyAsync(ybar, ynew, bytes, hipMemcpyDeviceToDevice, h->st));
@@ -874,11 +1066,16 @@ extern "C" int dmd_scatt_adjoint_rk4(dmd_scatt *h, double t0, double dt, int64_t
     }
     if (tiles && (rc = fold_G())) return rc;
     // dtheta_c = prefac_c / 2 Re <Gc, P_c>
-    if (gwords) DMD_HIP(hipMemsetAsync(tmp, 0, sizeof(double), h->st));
-    for (int cc = 0; gwords && cc < ncomp; cc++) {
-        if ((rc = launch_dot(h, gwords, Gc, comps[cc]->d_P, (double *)tmp))) return rc;
-        hipLaunchKernelGGL(k_take_scaled, dim3(1), dim3(64), 0, h->st, (double *)tmp, 0.5 * comps[cc]->prefac,
-                           d_dth + cc);
+    for (int c0 = 0; gwords && c0 < ncomp; c0 += kDots) {
+        DotArgs D{};
+        D.n = std::min(kDots, ncomp - c0);
+        for (int cc = 0; cc < D.n; cc++) {
+            D.p[cc] = comps[c0 + cc]->d_P;
+            D.scale[cc] = 0.5 * comps[c0 + cc]->prefac;
+        }
+        const int nparts = (int)std::min<int64_t>(1024, std::max<int64_t>(1, nblk(gwords, 256)));
+        hipLaunchKernelGGL(k_dots_partial, dim3(nparts), dim3(256), 0, h->st, gwords, Gc, D, h->d_dotpart);
+        hipLaunchKernelGGL(k_dots_final, dim3(D.n), dim3(256), 0, h->st, nparts, h->d_dotpart, D, d_dth + c0);
     }
     DMD_HIP(hipGetLastError());
     DMD_HIP(hipStreamSynchronize(h->st));
