@@ -534,12 +534,26 @@ __global__ __launch_bounds__(256) void k_dP_term(int64_t n, int nb, const double
 // order), so the lanes of a granule read one element's values together.  The
 // lane rebuilds its pair's dense P1, P2 in registers (zeros where absent) and
 // runs the dense GEMVs.
+// Bound by the stream of records, 32 loads of 16 bytes per lane in flight, so
+// by the wavefronts that the registers leave room for and by what keeps them
+// from their next loads.  Each side's row is summed into LDS as soon as it is
+// formed (holding both rows' increments to the end of the iteration costs 3 to
+// 8 %).  EARLY, the forms with an explicit 1 - rho or a compressed P: the first
+// pairs' records (and the row of their k) are on their way before the block
+// stages its rows and clears its accumulators, the next pairs' as soon as this
+// iteration's are used.  With DM1 that lets the rows be held in 236 registers
+// instead of 260 (two wavefronts per SIMD instead of one), and the compressed
+// form no longer spills.  The other two forms fetch where they use: they fit
+// two wavefronts per SIMD either way, and the early order costs them 1 to 9 %
+// (39.3 against 43.0 us at 443 k pairs).  Measured against the
+// former loop (records fetched where used in every form, 252 registers): 443 k pairs 42.4 -> 39.4 us,
+// 964 k 82.4 -> 79.9, 2.98 M 271 -> 264, 15.5 M 1272 -> 1263; DM1 991 k 106 ->
+// 101, 2.98 M 320 -> 311; compressed to 54 %, 58.2 M pairs 4.07 -> 4.00 ms.
 template <bool DM1, bool LIN, bool SP = false>
 __global__ __launch_bounds__(256, SP ? 2 : 1) void k_tiles_soa(int64_t nk, const double2 *__restrict__ P,
                                                    const uint32_t *__restrict__ pk,
                                                    const int64_t *__restrict__ cbeg,
                                                    const int32_t *__restrict__ clen, const int2 *__restrict__ cij,
-                                                   const int32_t *__restrict__ gbeg,
                                                    const double2 *__restrict__ rhoS,
                                                    const double2 *__restrict__ rho1S, double *__restrict__ hacc,
                                                    const uint32_t *__restrict__ pmask = nullptr,
@@ -547,199 +561,191 @@ __global__ __launch_bounds__(256, SP ? 2 : 1) void k_tiles_soa(int64_t nk, const
 {
     constexpr int NB2 = 4, NB4 = 16, EP = 32, R = DMD_TILE_R;  // nb = 2
     constexpr int W = 4, RPT = R / 256;  // rows per thread in the flush
+    constexpr bool EARLY = DM1 || SP;
     // LDS: Hermitian row increments of blocks I and J, structure of arrays
     // (double d of row r at d*R + r, conflict-free for the flush), and the
     // rho rows of block J, gathered per pair from LDS instead of L2.
     __shared__ double accA[4 * R], accB[4 * R];
     __shared__ double2 rhoJ[R * NB2];
-    const int c0 = gbeg[blockIdx.x], c1 = gbeg[blockIdx.x + 1];
-    const int I = cij[c0].x;
-    const int64_t I0 = (int64_t)I * R;
-    for (int i = threadIdx.x; i < 4 * R; i += blockDim.x) { accA[i] = 0.0; accB[i] = 0.0; }
+    const int c = blockIdx.x;
+    const int I = cij[c].x, J = cij[c].y;
+    const int64_t I0 = (int64_t)I * R, J0 = (int64_t)J * R;
+    const int64_t b = cbeg[c];
+    const int n = clen[c];
+    const int m = (n + 63) / 64;  // blocks of 64 slots; lane l owns chunk pairs l*m .. l*m+m-1
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    for (int c = c0; c < c1; c++) {
-        const int64_t b = cbeg[c];
-        const int n = clen[c];
-        const int m = (n + 63) / 64;  // blocks of 64 slots; lane l owns chunk pairs l*m .. l*m+m-1
-        const int J = cij[c].y;
-        const int64_t J0 = (int64_t)J * R;
-        double *aJ = (I == J) ? accA : accB;
-        if (!DM1) {
-            for (int i = threadIdx.x; i < R * NB2; i += blockDim.x)
-                rhoJ[i] = J0 * NB2 + i < nk * NB2 ? rhoS[J0 * NB2 + i] : make_double2(0, 0);
+    const int mq = (m + W - 1) / W;
+    const int i0 = wv * mq, i1 = min(m, i0 + mq);
+    auto code_of = [&](int it) {
+        return it < i1 && lane * m + it < n ? ld_stream(pk + b + (int64_t)it * 64 + lane) : 0u;
+    };
+    uint32_t code = 0u, code_next = code_of(i0);
+    // SP: the slot's mask and its granule's value offset, one iteration ahead
+    uint32_t mask_next = 0u, gofs_next = 0u;
+    auto sp_next = [&](int it) {
+        if (SP && it < i1) {
+            const int64_t s = b + (int64_t)it * 64 + lane;
+            mask_next = ld_stream(pmask + s);
+            gofs_next = ld_stream(gofs + (s >> 3));
         }
-        __syncthreads();
-        const int mq = (m + W - 1) / W;
-        const int i0 = wv * mq, i1 = min(m, i0 + mq);
-        uint32_t code_next = (i0 < i1 && lane * m + i0 < n) ? ld_stream(pk + b + (int64_t)i0 * 64 + lane) : 0u;
-        // SP: the slot's mask and its granule's value offset, one iteration ahead
-        uint32_t mask_next = 0u, gofs_next = 0u;
-        if (SP && i0 < i1) {
-            const int64_t s0 = b + (int64_t)i0 * 64 + lane;
-            mask_next = ld_stream(pmask + s0);
-            gofs_next = ld_stream(gofs + (s0 >> 3));
-        }
-        // rho of the lane's current row k: a lane walks a run of one k, so it is
-        // reloaded only where k changes
-        int lo1_cur = -1;
-        double2 rk[NB2], r1k[NB2];
+    };
+    sp_next(i0);
+    double2 p1[NB4], p2[NB4];
+    // rho of the lane's current row k: a lane walks a run of one k, so it is
+    // reloaded only where k changes
+    int lo1_cur = -1;
+    double2 rk[NB2], r1k[NB2];
 #pragma unroll
-        for (int q = 0; q < NB2; q++) { rk[q] = make_double2(0, 0); r1k[q] = make_double2(0, 0); }
-        for (int it = i0; it < i1; it++) {
-            const bool ok = lane * m + it < n;
-            // idle lanes read the chunk's first slot (always valid) and add
-            // nothing; with SP every lane keeps its own slot (a padding slot,
-            // mask 0, for idle lanes), so the 8 lanes of a granule are its 8 slots
-            const int64_t s = b + ((ok || SP) ? (int64_t)it * 64 + lane : 0);
-            const uint32_t code = code_next;
-            code_next = (it + 1 < i1 && lane * m + it + 1 < n) ? ld_stream(pk + b + (int64_t)(it + 1) * 64 + lane) : 0u;
-            uint32_t mask = 0u, vofs = 0u;
-            if (SP) {
-                mask = mask_next;
-                vofs = gofs_next;
-                if (it + 1 < i1) {
-                    const int64_t s1 = b + (int64_t)(it + 1) * 64 + lane;
-                    mask_next = ld_stream(pmask + s1);
-                    gofs_next = ld_stream(gofs + (s1 >> 3));
-                }
-            }
-            const int lo1 = code % R, lo2 = code / R;
-            const int64_t k = I0 + lo1, kp = J0 + lo2;
-            const double2 *g = P + (s >> 3) * (8 * EP) + (s & 7);
-            double2 rkp[NB2];
+    for (int q = 0; q < NB2; q++) { rk[q] = make_double2(0, 0); r1k[q] = make_double2(0, 0); }
+    // iteration it's code, row of k and records
+    auto fetch = [&](int it) {
+        const bool ok = lane * m + it < n;
+        code = code_next;
+        code_next = code_of(it + 1);
+        const int lo1 = code % R;
+        if (ok && lo1 != lo1_cur) {
 #pragma unroll
-            for (int q = 0; q < NB2; q++) rkp[q] = DM1 ? rhoS[kp * NB2 + q] : rhoJ[lo2 * NB2 + q];
-            if (ok && lo1 != lo1_cur) {
-#pragma unroll
-                for (int q = 0; q < NB2; q++) rk[q] = rhoS[k * NB2 + q];
-                if (DM1) {
-#pragma unroll
-                    for (int q = 0; q < NB2; q++) r1k[q] = rho1S[k * NB2 + q];
-                }
-                lo1_cur = lo1;
-            }
-            double2 r1kp[NB2];
+            for (int q = 0; q < NB2; q++) rk[q] = rhoS[(I0 + lo1) * NB2 + q];
             if (DM1) {
 #pragma unroll
-                for (int q = 0; q < NB2; q++) r1kp[q] = rho1S[kp * NB2 + q];
+                for (int q = 0; q < NB2; q++) r1k[q] = rho1S[(I0 + lo1) * NB2 + q];
             }
-            // 1-rho: explicit rows with DM1, else formed from rho where used
-            auto om_k = [&](int q) { return DM1 ? r1k[q] : one_minus(rk, q); };
-            auto om_kp = [&](int q) { return DM1 ? r1kp[q] : one_minus(rkp, q); };
-            const bool rev = ok && k < kp;
+            lo1_cur = lo1;
+        }
+        // idle lanes read the chunk's first slot (always valid) and add
+        // nothing; with SP every lane keeps its own slot (a padding slot,
+        // mask 0, for idle lanes), so the 8 lanes of a granule are its 8 slots
+        const int64_t s = b + ((ok || SP) ? (int64_t)it * 64 + lane : 0);
+        if (SP) {
+            // element-major values of the granule: for element el = 0 .. 31
+            // (P1 then P2) the values of the granule's slots that have it,
+            // in slot order.  One ballot per element gives each lane its
+            // place; an element a slot does not have is zero, so the dense
+            // GEMVs below run unchanged.
+            const uint32_t mask = mask_next;
+            const double2 *gv = P + gofs_next;
+            sp_next(it + 1);
+            const int gsh = lane & 56;
+            const uint32_t below = (1u << (lane & 7)) - 1u;
+            int base = 0;
+#pragma unroll
+            for (int el = 0; el < 2 * NB4; el++) {
+                const bool has = (mask >> el) & 1u;
+                const uint32_t gb = (uint32_t)(__ballot(has) >> gsh) & 0xffu;
+                double2 v = make_double2(0, 0);
+                if (has) v = ld_stream(gv + base + __popc(gb & below));
+                base += __popc(gb);
+                if (el < NB4) p1[el] = v;
+                else p2[el - NB4] = v;
+            }
+        } else {
+            const double2 *g = P + (s >> 3) * (8 * EP) + (s & 7);
+#pragma unroll
+            for (int el = 0; el < NB4; el++) p1[el] = ld_stream(g + el * 8);
+#pragma unroll
+            for (int el = 0; el < NB4; el++) p2[el] = ld_stream(g + (NB4 + el) * 8);
+        }
+    };
+    if (EARLY && i0 < i1) fetch(i0);
+    for (int i = threadIdx.x; i < 4 * R; i += blockDim.x) { accA[i] = 0.0; accB[i] = 0.0; }
+    if (!DM1) {
+        for (int i = threadIdx.x; i < R * NB2; i += blockDim.x)
+            rhoJ[i] = J0 * NB2 + i < nk * NB2 ? rhoS[J0 * NB2 + i] : make_double2(0, 0);
+    }
+    double *aJ = (I == J) ? accA : accB;
+    __syncthreads();
+    for (int it = i0; it < i1;) {
+        if (!EARLY) fetch(it);
+        const bool ok = lane * m + it < n;
+        const int lo1 = code % R, lo2 = code / R;
+        const int64_t kp = J0 + lo2;
+        const bool rev = ok && I0 + lo1 < kp;
+        double2 rkp[NB2];
+#pragma unroll
+        for (int q = 0; q < NB2; q++) rkp[q] = DM1 ? rhoS[kp * NB2 + q] : rhoJ[lo2 * NB2 + q];
+        double2 r1kp[NB2];
+        if (DM1) {
+#pragma unroll
+            for (int q = 0; q < NB2; q++) r1kp[q] = rho1S[kp * NB2 + q];
+        }
+        // 1-rho: explicit rows with DM1, else formed from rho where used
+        auto om_k = [&](int q) { return DM1 ? r1k[q] : one_minus(rk, q); };
+        auto om_kp = [&](int q) { return DM1 ? r1kp[q] : one_minus(rkp, q); };
+        auto add_k = [&](const double *hf) {
+            if (ok) {
+#pragma unroll
+                for (int d = 0; d < 4; d++) atomicAdd(&accA[d * R + lo1], hf[d]);
+            }
+        };
+        auto add_kp = [&](const double *hr) {
+            if (rev) {
+#pragma unroll
+                for (int d = 0; d < 4; d++) atomicAdd(&aJ[d * R + lo2], hr[d]);
+            }
+        };
+        double hf[4], hr[4];
+        if (LIN) {
+            double2 x[NB2], y[NB2];
+#pragma unroll
+            for (int i = 0; i < NB2; i++) {
+                x[i] = make_double2(0, 0);
+                y[i] = make_double2(0, 0);
+#pragma unroll
+                for (int q = 0; q < NB2; q++) {
+                    cfma(x[i], p1[i * NB2 + q], rkp[q]);  // X_k[i]  += Lscij[i,q] drho_k'[q]
+                    cfma(y[i], p2[i * NB2 + q], rk[q]);   // Y_k'[i] += Lscji[i,q] drho_k[q]
+                }
+            }
+            herm_of(x, hf);
+            herm_of(y, hr);
+            add_k(hf);
+            add_kp(hr);
+        } else {
             // forward Pdm_k = P1 rho_k', dm1P_k = (1-rho_k')^T P2 (f1, f2);
             // reverse Pdm_k' = conj(P2) rho_k, dm1P_k' = (1-rho_k)^T conj(P1) (g1, g2)
             double2 f1[NB2], f2[NB2], g1[NB2], g2[NB2];
-            double2 p1[NB4], p2[NB4];
-            if (SP) {
-                // element-major values of the granule: for element el = 0 .. 31
-                // (P1 then P2) the values of the granule's slots that have it,
-                // in slot order.  One ballot per element gives each lane its
-                // place; an element a slot does not have is zero, so the dense
-                // GEMVs below run unchanged.
-                const double2 *gv = P + vofs;
-                const int gsh = lane & 56;
-                const uint32_t below = (1u << (lane & 7)) - 1u;
-                int base = 0;
 #pragma unroll
-                for (int el = 0; el < 2 * NB4; el++) {
-                    const bool has = (mask >> el) & 1u;
-                    const uint32_t gb = (uint32_t)(__ballot(has) >> gsh) & 0xffu;
-                    double2 v = make_double2(0, 0);
-                    if (has) v = ld_stream(gv + base + __popc(gb & below));
-                    base += __popc(gb);
-                    if (el < NB4) p1[el] = v;
-                    else p2[el - NB4] = v;
-                }
-            } else {
+            for (int i = 0; i < NB2; i++) {
+                f1[i] = make_double2(0, 0);
+                f2[i] = make_double2(0, 0);
 #pragma unroll
-                for (int el = 0; el < NB4; el++) p1[el] = ld_stream(g + el * 8);
-#pragma unroll
-                for (int el = 0; el < NB4; el++) p2[el] = ld_stream(g + (NB4 + el) * 8);
-            }
-            {
-                if (LIN) {
-                    double2 x[NB2], y[NB2];
-#pragma unroll
-                    for (int i = 0; i < NB2; i++) {
-                        x[i] = make_double2(0, 0);
-                        y[i] = make_double2(0, 0);
-#pragma unroll
-                        for (int q = 0; q < NB2; q++) {
-                            cfma(x[i], p1[i * NB2 + q], rkp[q]);  // X_k[i]  += Lscij[i,q] drho_k'[q]
-                            cfma(y[i], p2[i * NB2 + q], rk[q]);   // Y_k'[i] += Lscji[i,q] drho_k[q]
-                        }
-                    }
-                    double hf[4], hr[4];
-                    herm_of(x, hf);
-                    herm_of(y, hr);
-                    if (ok) {
-#pragma unroll
-                        for (int d = 0; d < 4; d++) atomicAdd(&accA[d * R + lo1], hf[d]);
-                    }
-                    if (rev) {
-#pragma unroll
-                        for (int d = 0; d < 4; d++) atomicAdd(&aJ[d * R + lo2], hr[d]);
-                    }
-                    continue;
-                }
-                // forward (row k)
-                {
-#pragma unroll
-                    for (int i = 0; i < NB2; i++) {
-                        f1[i] = make_double2(0, 0);
-                        f2[i] = make_double2(0, 0);
-#pragma unroll
-                        for (int q = 0; q < NB2; q++) {
-                            cfma(f1[i], p1[i * NB2 + q], rkp[q]);      // Pdm_k[i]  += P1[i,q] rho_k'[q]
-                            cfma(f2[i], om_kp(q), p2[q * NB2 + i]);    // dm1P_k[i] += (1-rho_k')[q] P2[q,i]
-                        }
-                    }
-                    double hf[4];
-                    herm_inc(f1, f2, rk, DM1 ? r1k : nullptr, hf);
-                    if (ok) {
-#pragma unroll
-                        for (int d = 0; d < 4; d++) atomicAdd(&accA[d * R + lo1], hf[d]);
-                    }
-                }
-                // reverse (row k')
-                {
-#pragma unroll
-                    for (int i = 0; i < NB2; i++) {
-                        g1[i] = make_double2(0, 0);
-                        g2[i] = make_double2(0, 0);
-#pragma unroll
-                        for (int q = 0; q < NB2; q++) {
-                            cfmac(g1[i], rk[q], p2[i * NB2 + q]);      // Pdm_k'[i]  += rho_k[q] conj(P2[i,q])
-                            cfmac(g2[i], om_k(q), p1[q * NB2 + i]);    // dm1P_k'[i] += (1-rho_k)[q] conj(P1[q,i])
-                        }
-                    }
-                    double hr[4];
-                    herm_inc(g1, g2, rkp, DM1 ? r1kp : nullptr, hr);
-                    if (rev) {
-#pragma unroll
-                        for (int d = 0; d < 4; d++) atomicAdd(&aJ[d * R + lo2], hr[d]);
-                    }
+                for (int q = 0; q < NB2; q++) {
+                    cfma(f1[i], p1[i * NB2 + q], rkp[q]);      // Pdm_k[i]  += P1[i,q] rho_k'[q]
+                    cfma(f2[i], om_kp(q), p2[q * NB2 + i]);    // dm1P_k[i] += (1-rho_k')[q] P2[q,i]
                 }
             }
+            herm_inc(f1, f2, rk, DM1 ? r1k : nullptr, hf);
+            add_k(hf);
+#pragma unroll
+            for (int i = 0; i < NB2; i++) {
+                g1[i] = make_double2(0, 0);
+                g2[i] = make_double2(0, 0);
+#pragma unroll
+                for (int q = 0; q < NB2; q++) {
+                    cfmac(g1[i], rk[q], p2[i * NB2 + q]);      // Pdm_k'[i]  += rho_k[q] conj(P2[i,q])
+                    cfmac(g2[i], om_k(q), p1[q * NB2 + i]);    // dm1P_k'[i] += (1-rho_k)[q] conj(P1[q,i])
+                }
+            }
+            herm_inc(g1, g2, rkp, DM1 ? r1kp : nullptr, hr);
+            add_kp(hr);
         }
-        __syncthreads();  // block J done
-        if (I != J) {  // flush and clear block J
-#pragma unroll
-            for (int t = 0; t < RPT; t++) {
-                const int r = t * 256 + threadIdx.x;
-                double hv[4];
-#pragma unroll
-                for (int d = 0; d < 4; d++) { hv[d] = accB[d * R + r]; accB[d * R + r] = 0.0; }
-                flush_herm_wave(hv, lane, J0 + (r & ~63), nk, hacc);
-            }
+        if (++it >= i1) break;
+        if (EARLY) {
+            // not before the sums: two record sets live at once would cost a wave per SIMD
+            __builtin_amdgcn_sched_barrier(0);
+            fetch(it);
         }
-        __syncthreads();  // rhoJ and accB free for the next chunk
     }
+    __syncthreads();
 #pragma unroll
     for (int t = 0; t < RPT; t++) {
         const int r = t * 256 + threadIdx.x;
         double hv[4];
+        if (I != J) {
+#pragma unroll
+            for (int d = 0; d < 4; d++) hv[d] = accB[d * R + r];
+            flush_herm_wave(hv, lane, J0 + (r & ~63), nk, hacc);
+        }
 #pragma unroll
         for (int d = 0; d < 4; d++) hv[d] = accA[d * R + r];
         flush_herm_wave(hv, lane, I0 + (r & ~63), nk, hacc);
@@ -1733,22 +1739,22 @@ static void launch_tiles_sums(dmd_scatt *h, bool dm1)
 {
     if (h->ngroups > 0) {
         if (h->linear)
-            hipLaunchKernelGGL((k_tiles_soa<false, true>), dim3((unsigned)h->ngroups), dim3(256), 0, h->st, h->nk, h->d_P,
-                               h->d_pk, h->d_cbeg, h->d_clen, h->d_cij, h->d_gbeg, h->d_rhoS, h->d_rho1S, h->d_acc_herm);
+            hipLaunchKernelGGL((k_tiles_soa<false, true>), dim3((unsigned)h->nchunks), dim3(256), 0, h->st, h->nk, h->d_P,
+                               h->d_pk, h->d_cbeg, h->d_clen, h->d_cij, h->d_rhoS, h->d_rho1S, h->d_acc_herm);
         else if (h->d_spv && dm1)
-            hipLaunchKernelGGL((k_tiles_soa<true, false, true>), dim3((unsigned)h->ngroups), dim3(256), 0, h->st, h->nk,
-                               h->d_spv, h->d_pk, h->d_cbeg, h->d_clen, h->d_cij, h->d_gbeg, h->d_rhoS, h->d_rho1S,
+            hipLaunchKernelGGL((k_tiles_soa<true, false, true>), dim3((unsigned)h->nchunks), dim3(256), 0, h->st, h->nk,
+                               h->d_spv, h->d_pk, h->d_cbeg, h->d_clen, h->d_cij, h->d_rhoS, h->d_rho1S,
                                h->d_acc_herm, h->d_spmask, h->d_spgofs);
         else if (h->d_spv)
-            hipLaunchKernelGGL((k_tiles_soa<false, false, true>), dim3((unsigned)h->ngroups), dim3(256), 0, h->st, h->nk,
-                               h->d_spv, h->d_pk, h->d_cbeg, h->d_clen, h->d_cij, h->d_gbeg, h->d_rhoS, h->d_rho1S,
+            hipLaunchKernelGGL((k_tiles_soa<false, false, true>), dim3((unsigned)h->nchunks), dim3(256), 0, h->st, h->nk,
+                               h->d_spv, h->d_pk, h->d_cbeg, h->d_clen, h->d_cij, h->d_rhoS, h->d_rho1S,
                                h->d_acc_herm, h->d_spmask, h->d_spgofs);
         else if (dm1)
-            hipLaunchKernelGGL((k_tiles_soa<true, false>), dim3((unsigned)h->ngroups), dim3(256), 0, h->st, h->nk, h->d_P,
-                               h->d_pk, h->d_cbeg, h->d_clen, h->d_cij, h->d_gbeg, h->d_rhoS, h->d_rho1S, h->d_acc_herm);
+            hipLaunchKernelGGL((k_tiles_soa<true, false>), dim3((unsigned)h->nchunks), dim3(256), 0, h->st, h->nk, h->d_P,
+                               h->d_pk, h->d_cbeg, h->d_clen, h->d_cij, h->d_rhoS, h->d_rho1S, h->d_acc_herm);
         else
-            hipLaunchKernelGGL((k_tiles_soa<false, false>), dim3((unsigned)h->ngroups), dim3(256), 0, h->st, h->nk, h->d_P,
-                               h->d_pk, h->d_cbeg, h->d_clen, h->d_cij, h->d_gbeg, h->d_rhoS, h->d_rho1S, h->d_acc_herm);
+            hipLaunchKernelGGL((k_tiles_soa<false, false>), dim3((unsigned)h->nchunks), dim3(256), 0, h->st, h->nk, h->d_P,
+                               h->d_pk, h->d_cbeg, h->d_clen, h->d_cij, h->d_rhoS, h->d_rho1S, h->d_acc_herm);
     }
 }
 
