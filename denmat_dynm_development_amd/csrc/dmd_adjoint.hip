@@ -258,177 +258,213 @@ __global__ void k_vjp_stage_in(int64_t nk, const double2 *__restrict__ rho, cons
         for (int j = 0; j < NB; j++) uS[k * NB2 + i * NB + j] = cadd(vs[i * NB + j], cconj(vs[j * NB + i]));
 }
 
-// 2 x 2 products of the VJP: X' = u r, Y' = (1 - r) u
-__device__ __forceinline__ void xy_of(const double2 *r, const double2 *u, double2 *x, double2 *y)
+// 2 x 2 products of the VJP: X' = u r and Y' = (1 - r) u
+__device__ __forceinline__ void x_of(const double2 *r, const double2 *u, double2 *x)
 {
 #pragma unroll
     for (int i = 0; i < 2; i++)
 #pragma unroll
         for (int j = 0; j < 2; j++) {
-            double2 p = make_double2(0, 0), q = make_double2(0, 0);
+            x[i * 2 + j] = make_double2(0, 0);
 #pragma unroll
-            for (int m = 0; m < 2; m++) {
-                cfma(p, u[i * 2 + m], r[m * 2 + j]);
-                cfma(q, one_minus(r, i * 2 + m), u[m * 2 + j]);
-            }
-            x[i * 2 + j] = p;
-            y[i * 2 + j] = q;
+            for (int m = 0; m < 2; m++) cfma(x[i * 2 + j], u[i * 2 + m], r[m * 2 + j]);
         }
 }
-// packed Hermitian part of s - (u F1^+ + F2^+ u) (2 x 2)
-__device__ __forceinline__ void vjp_row_inc(const double2 *s, const double2 *u, const double2 *F1, const double2 *F2,
-                                            double hv[4])
+__device__ __forceinline__ void y_of(const double2 *r, const double2 *u, double2 *y)
 {
-    double2 x[4];
 #pragma unroll
     for (int i = 0; i < 2; i++)
 #pragma unroll
         for (int j = 0; j < 2; j++) {
-            double2 g = s[i * 2 + j];
+            y[i * 2 + j] = make_double2(0, 0);
+#pragma unroll
+            for (int m = 0; m < 2; m++) cfma(y[i * 2 + j], one_minus(r, i * 2 + m), u[m * 2 + j]);
+        }
+}
+// c -= u F1^+ (2 x 2)
+__device__ __forceinline__ void sub_u_f1(double2 *c, const double2 *u, const double2 *f1)
+{
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
 #pragma unroll
             for (int m = 0; m < 2; m++) {
-                const double2 a = cmulc(u[i * 2 + m], F1[j * 2 + m]);        // (u F1^+)_ij
-                const double2 b = cmul(cconj(F2[m * 2 + i]), u[m * 2 + j]);  // (F2^+ u)_ij
-                g = make_double2(g.x - a.x - b.x, g.y - a.y - b.y);
+                const double2 a = cmulc(u[i * 2 + m], f1[j * 2 + m]);
+                c[i * 2 + j] = csub(c[i * 2 + j], a);
             }
-            x[i * 2 + j] = g;
-        }
-    herm_of(x, hv);
+}
+// c -= F2^+ u (2 x 2)
+__device__ __forceinline__ void sub_f2_u(double2 *c, const double2 *u, const double2 *f2)
+{
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int m = 0; m < 2; m++) {
+                const double2 b = cmul(cconj(f2[m * 2 + i]), u[m * 2 + j]);
+                c[i * 2 + j] = csub(c[i * 2 + j], b);
+            }
 }
 
-__global__ __launch_bounds__(256) void k_tiles_vjp(int64_t nk, const double2 *__restrict__ P,
+// Bound by the stream of records (512 B per pair): the time is set by the
+// loads in flight.  One block of 8 wavefronts per CU, two per SIMD, because the
+// rows of block J (rho_S and u_S) and both blocks' increments take 96 of the
+// 160 KB of LDS.  The two per SIMD leave a lane 256 registers, 128 of them its
+// record: each product is formed and folded before the next (a row's X', Y' too,
+// rather than kept along the run), u's lower element is the conjugate of the
+// upper one, and a chunk's addresses are 32-bit offsets from its own start
+// (chunks begin on multiples of 64 slots).  Blocks of 4 wavefronts holding X', Y'
+// took 340 registers, one wavefront per SIMD: 66 us at 477 k pairs against 49
+// (5.0 TB/s), the forward contraction of the same pairs being 44.
+__global__ __launch_bounds__(512) void k_tiles_vjp(int64_t nk, const double2 *__restrict__ P,
                                                    const uint32_t *__restrict__ pk, const int64_t *__restrict__ cbeg,
                                                    const int32_t *__restrict__ clen, const int2 *__restrict__ cij,
-                                                   const int32_t *__restrict__ gbeg, const double2 *__restrict__ rS,
-                                                   const double2 *__restrict__ uS, double *__restrict__ hacc)
+                                                   const double2 *__restrict__ rS, const double2 *__restrict__ uS,
+                                                   double *__restrict__ hacc)
 {
     constexpr int NB2 = 4, NB4 = 16, EP = 32, R = DMD_TILE_R;
-    constexpr int W = 4, RPT = R / 256;
+    constexpr int W = 8, RPT = R / 512;
     __shared__ double accA[4 * R], accB[4 * R];
     __shared__ double2 rJ[R * NB2], uJ[R * NB2];
-    const int c0 = gbeg[blockIdx.x], c1 = gbeg[blockIdx.x + 1];
-    const int I = cij[c0].x;
-    const int64_t I0 = (int64_t)I * R;
-    for (int i = threadIdx.x; i < 4 * R; i += blockDim.x) { accA[i] = 0.0; accB[i] = 0.0; }
+    const int I = cij[blockIdx.x].x, J = cij[blockIdx.x].y;
+    const int64_t I0 = (int64_t)I * R, J0 = (int64_t)J * R;
+    const int64_t b = cbeg[blockIdx.x];
+    const int n = clen[blockIdx.x];
+    const int m = (n + 63) / 64;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    for (int c = c0; c < c1; c++) {
-        const int64_t b = cbeg[c];
-        const int n = clen[c];
-        const int m = (n + 63) / 64;
-        const int J = cij[c].y;
-        const int64_t J0 = (int64_t)J * R;
-        double *aJ = (I == J) ? accA : accB;
-        for (int i = threadIdx.x; i < R * NB2; i += blockDim.x) {
-            const bool in = J0 * NB2 + i < nk * NB2;
-            rJ[i] = in ? rS[J0 * NB2 + i] : make_double2(0, 0);
-            uJ[i] = in ? uS[J0 * NB2 + i] : make_double2(0, 0);
+    const int mq = (m + W - 1) / W;
+    const int i0 = wv * mq, i1 = min(m, i0 + mq);
+    for (int i = threadIdx.x; i < 4 * R; i += blockDim.x) { accA[i] = 0.0; accB[i] = 0.0; }
+    for (int i = threadIdx.x; i < R * NB2; i += blockDim.x) {
+        const bool in = J0 * NB2 + i < nk * NB2;
+        rJ[i] = in ? rS[J0 * NB2 + i] : make_double2(0, 0);
+        uJ[i] = in ? uS[J0 * NB2 + i] : make_double2(0, 0);
+    }
+    double *aJ = (I == J) ? accA : accB;
+    __syncthreads();
+    uint32_t code_next = (i0 < i1 && lane * m + i0 < n) ? ld_stream(pk + b + (int64_t)i0 * 64 + lane) : 0u;
+    const double2 *rI = rS + I0 * NB2, *uI = uS + I0 * NB2;
+    const double2 *Pc = P + (b >> 3) * (8 * EP);
+    int lo1_cur = -1;
+    double2 rk[NB2], uk[NB2];
+#pragma unroll
+    for (int q = 0; q < NB2; q++) { rk[q] = make_double2(0, 0); uk[q] = make_double2(0, 0); }
+    for (int it = i0; it < i1; it++) {
+        const bool ok = lane * m + it < n;
+        const int sl = ok ? it * 64 + lane : 0;
+        const uint32_t code = code_next;
+        code_next = (it + 1 < i1 && lane * m + it + 1 < n) ? ld_stream(pk + b + (int64_t)(it + 1) * 64 + lane) : 0u;
+        const int lo1 = code % R, lo2 = code / R;
+        const double2 *g = Pc + (sl >> 3) * (8 * EP) + (sl & 7);
+        if (ok && lo1 != lo1_cur) {
+#pragma unroll
+            for (int q = 0; q < NB2; q++) { rk[q] = rI[lo1 * NB2 + q]; if (q != 2) uk[q] = uI[lo1 * NB2 + q]; }
+            lo1_cur = lo1;
         }
-        __syncthreads();
-        const int mq = (m + W - 1) / W;
-        const int i0 = wv * mq, i1 = min(m, i0 + mq);
-        uint32_t code_next = (i0 < i1 && lane * m + i0 < n) ? ld_stream(pk + b + (int64_t)i0 * 64 + lane) : 0u;
-        int lo1_cur = -1;
-        double2 rk[NB2], uk[NB2], xk[NB2], yk[NB2];
+        uk[2] = cconj(uk[1]);
+        const bool diag = I == J && lo1 == lo2, rev = ok && (I < J || (I == J && lo1 < lo2));
+        double2 p1[NB4], p2[NB4];
 #pragma unroll
-        for (int q = 0; q < NB2; q++) {
-            rk[q] = make_double2(0, 0); uk[q] = make_double2(0, 0);
-            xk[q] = make_double2(0, 0); yk[q] = make_double2(0, 0);
-        }
-        for (int it = i0; it < i1; it++) {
-            const bool ok = lane * m + it < n;
-            const int64_t s = b + (ok ? (int64_t)it * 64 + lane : 0);
-            const uint32_t code = code_next;
-            code_next = (it + 1 < i1 && lane * m + it + 1 < n) ? ld_stream(pk + b + (int64_t)(it + 1) * 64 + lane) : 0u;
-            const int lo1 = code % R, lo2 = code / R;
-            const int64_t k = I0 + lo1, kp = J0 + lo2;
-            const double2 *g = P + (s >> 3) * (8 * EP) + (s & 7);
-            double2 rp[NB2], up[NB2], xp[NB2], yp[NB2];
+        for (int el = 0; el < NB4; el++) p1[el] = ld_stream(g + el * 8);
 #pragma unroll
-            for (int q = 0; q < NB2; q++) { rp[q] = rJ[lo2 * NB2 + q]; up[q] = uJ[lo2 * NB2 + q]; }
-            xy_of(rp, up, xp, yp);
-            if (ok && lo1 != lo1_cur) {
-#pragma unroll
-                for (int q = 0; q < NB2; q++) { rk[q] = rS[k * NB2 + q]; uk[q] = uS[k * NB2 + q]; }
-                xy_of(rk, uk, xk, yk);
-                lo1_cur = lo1;
-            }
-            const bool diag = k == kp, rev = ok && k < kp;
-            double2 p1[NB4], p2[NB4];
-#pragma unroll
-            for (int el = 0; el < NB4; el++) p1[el] = ld_stream(g + el * 8);
-#pragma unroll
-            for (int el = 0; el < NB4; el++) p2[el] = ld_stream(g + (NB4 + el) * 8);
-            // the reverse-form partner term conj(P2) X'_k + P1^H Y'_k: row k' of a
-            // k < k' pair, and row k of a k = k' pair
-            double2 sr[NB2];
+        for (int el = 0; el < NB4; el++) p2[el] = ld_stream(g + (NB4 + el) * 8);
+        // the reverse-form partner term conj(P2) X'_k + P1^H Y'_k: row k' of a
+        // k < k' pair, and row k of a k = k' pair
+        double2 sr[NB2];
+        {
+            double2 f[NB2];
+            x_of(rk, uk, f);
 #pragma unroll
             for (int i = 0; i < NB2; i++) {
                 sr[i] = make_double2(0, 0);
 #pragma unroll
-                for (int q = 0; q < NB2; q++) {
-                    cfmac(sr[i], xk[q], p2[i * NB2 + q]);
-                    cfmac(sr[i], yk[q], p1[q * NB2 + i]);
-                }
+                for (int q = 0; q < NB2; q++) cfmac(sr[i], f[q], p2[i * NB2 + q]);
             }
-            {  // forward direction, row k
-                double2 f1[NB2], f2[NB2], sf[NB2];
+            y_of(rk, uk, f);
 #pragma unroll
-                for (int i = 0; i < NB2; i++) {
-                    f1[i] = make_double2(0, 0);
-                    f2[i] = make_double2(0, 0);
-                    sf[i] = make_double2(0, 0);
+            for (int i = 0; i < NB2; i++)
 #pragma unroll
-                    for (int q = 0; q < NB2; q++) {
-                        cfma(f1[i], p1[i * NB2 + q], rp[q]);         // P1 rho_k'
-                        cfma(f2[i], one_minus(rp, q), p2[q * NB2 + i]);  // (1 - rho_k')^T P2
-                        cfma(sf[i], p1[i * NB2 + q], xp[q]);         // P1 X'_k'
-                        cfma(sf[i], yp[q], p2[q * NB2 + i]);         // P2^T Y'_k'
-                    }
-                }
-                double hf[4];
-                vjp_row_inc(diag ? sr : sf, uk, f1, f2, hf);
-                if (ok) {
+                for (int q = 0; q < NB2; q++) cfmac(sr[i], f[q], p1[q * NB2 + i]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        {  // forward direction, row k
+            double2 sf[NB2], f[NB2], rp[NB2];
 #pragma unroll
-                    for (int d = 0; d < 4; d++) atomicAdd(&accA[d * R + lo1], hf[d]);
-                }
+            for (int q = 0; q < NB2; q++) rp[q] = rJ[lo2 * NB2 + q];
+            x_of(rp, uJ + lo2 * NB2, f);
+#pragma unroll
+            for (int i = 0; i < NB2; i++) {
+                sf[i] = make_double2(0, 0);
+#pragma unroll
+                for (int q = 0; q < NB2; q++) cfma(sf[i], p1[i * NB2 + q], f[q]);  // P1 X'_k'
             }
-            {  // reverse direction, row k'
-                double2 g1[NB2], g2[NB2];
+            y_of(rp, uJ + lo2 * NB2, f);
 #pragma unroll
-                for (int i = 0; i < NB2; i++) {
-                    g1[i] = make_double2(0, 0);
-                    g2[i] = make_double2(0, 0);
+            for (int i = 0; i < NB2; i++) {
 #pragma unroll
-                    for (int q = 0; q < NB2; q++) {
-                        cfmac(g1[i], rk[q], p2[i * NB2 + q]);             // conj(P2) rho_k
-                        cfmac(g2[i], one_minus(rk, q), p1[q * NB2 + i]);  // (1 - rho_k)^T conj(P1)
-                    }
-                }
-                double hr[4];
-                vjp_row_inc(sr, up, g1, g2, hr);
-                if (rev) {
+                for (int q = 0; q < NB2; q++) cfma(sf[i], f[q], p2[q * NB2 + i]);  // P2^T Y'_k'
+                if (diag) sf[i] = sr[i];
+            }
 #pragma unroll
-                    for (int d = 0; d < 4; d++) atomicAdd(&aJ[d * R + lo2], hr[d]);
-                }
+            for (int i = 0; i < NB2; i++) {
+                f[i] = make_double2(0, 0);
+#pragma unroll
+                for (int q = 0; q < NB2; q++) cfma(f[i], p1[i * NB2 + q], rp[q]);  // P1 rho_k'
+            }
+            sub_u_f1(sf, uk, f);
+#pragma unroll
+            for (int i = 0; i < NB2; i++) {
+                f[i] = make_double2(0, 0);
+#pragma unroll
+                for (int q = 0; q < NB2; q++) cfma(f[i], one_minus(rp, q), p2[q * NB2 + i]);  // (1 - rho_k')^T P2
+            }
+            sub_f2_u(sf, uk, f);
+            double hf[4];
+            herm_of(sf, hf);
+            if (ok) {
+#pragma unroll
+                for (int d = 0; d < 4; d++) atomicAdd(&accA[d * R + lo1], hf[d]);
             }
         }
-        __syncthreads();
-        if (I != J) {
+        __builtin_amdgcn_sched_barrier(0);
+        {  // reverse direction, row k'
+            double2 f[NB2], up[NB2];
 #pragma unroll
-            for (int t = 0; t < RPT; t++) {
-                const int r = t * 256 + threadIdx.x;
-                double hv[4];
+            for (int q = 0; q < NB2; q++) up[q] = uJ[lo2 * NB2 + q];
 #pragma unroll
-                for (int d = 0; d < 4; d++) { hv[d] = accB[d * R + r]; accB[d * R + r] = 0.0; }
-                flush_herm_wave(hv, lane, J0 + (r & ~63), nk, hacc);
+            for (int i = 0; i < NB2; i++) {
+                f[i] = make_double2(0, 0);
+#pragma unroll
+                for (int q = 0; q < NB2; q++) cfmac(f[i], rk[q], p2[i * NB2 + q]);  // conj(P2) rho_k
+            }
+            sub_u_f1(sr, up, f);
+#pragma unroll
+            for (int i = 0; i < NB2; i++) {
+                f[i] = make_double2(0, 0);
+#pragma unroll
+                for (int q = 0; q < NB2; q++) cfmac(f[i], one_minus(rk, q), p1[q * NB2 + i]);  // (1 - rho_k)^T conj(P1)
+            }
+            sub_f2_u(sr, up, f);
+            double hr[4];
+            herm_of(sr, hr);
+            if (rev) {
+#pragma unroll
+                for (int d = 0; d < 4; d++) atomicAdd(&aJ[d * R + lo2], hr[d]);
             }
         }
-        __syncthreads();
     }
+    __syncthreads();
 #pragma unroll
     for (int t = 0; t < RPT; t++) {
-        const int r = t * 256 + threadIdx.x;
+        const int r = t * 512 + threadIdx.x;
         double hv[4];
+        if (I != J) {
+#pragma unroll
+            for (int d = 0; d < 4; d++) hv[d] = accB[d * R + r];
+            flush_herm_wave(hv, lane, J0 + (r & ~63), nk, hacc);
+        }
 #pragma unroll
         for (int d = 0; d < 4; d++) hv[d] = accA[d * R + r];
         flush_herm_wave(hv, lane, I0 + (r & ~63), nk, hacc);
@@ -592,8 +628,10 @@ __global__ __launch_bounds__(256) void k_adj_G(int64_t nslots, const int32_t *__
             rp[q] = rS[st * stride + bk * NB2 + q];
             up[q] = uS[st * stride + bk * NB2 + q];
         }
-        xy_of(rk, uk, xk, yk);
-        xy_of(rp, up, xp, yp);
+        x_of(rk, uk, xk);
+        y_of(rk, uk, yk);
+        x_of(rp, up, xp);
+        y_of(rp, up, yp);
 #pragma unroll
         for (int mm = 0; mm < NB2; mm++)
 #pragma unroll
@@ -727,9 +765,9 @@ static int launch_vjp_nb(dmd_scatt *h, const double2 *y, const double2 *v, doubl
 // the tile VJP's pass alone on prepared operands: packed rows into d_acc_herm
 static int launch_vjp_pass(dmd_scatt *h, const double2 *rS, const double2 *uS)
 {
-    if (h->ngroups > 0)
-        hipLaunchKernelGGL(k_tiles_vjp, dim3((unsigned)h->ngroups), dim3(256), 0, h->st, h->nk, h->d_P, h->d_pk,
-                           h->d_cbeg, h->d_clen, h->d_cij, h->d_gbeg, rS, uS, h->d_acc_herm);
+    if (h->nchunks > 0)
+        hipLaunchKernelGGL(k_tiles_vjp, dim3((unsigned)h->nchunks), dim3(512), 0, h->st, h->nk, h->d_P, h->d_pk,
+                           h->d_cbeg, h->d_clen, h->d_cij, rS, uS, h->d_acc_herm);
     DMD_HIP(hipGetLastError());
     return DMD_OK;
 }

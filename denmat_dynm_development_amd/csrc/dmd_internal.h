@@ -31,11 +31,8 @@ inline unsigned nblk(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); 
 
 // rows per tile of the tile kernel (a multiple of 256)
 #define DMD_TILE_R 512
-// chunks of one row block a tile-kernel workgroup takes in sequence
-#define DMD_TILE_GROUP 1
 // nb = 4 panel kernel: rows per panel, pairs per chunk (one workgroup) at most
 #define DMD_TILE4_R 32
-#define DMD_TILE4_GROUP 1
 #define DMD_TILE4_CMAX 2048
 // what a workgroup's prologue and flush cost, in pairs of its stream (the
 // chunk planner's weights; from sweeps of the chunk length)
@@ -226,8 +223,7 @@ struct dmd_scatt {
     int64_t *d_cbeg = nullptr;           // tile chunks: first pair, length, tile (I, J)
     int32_t *d_clen = nullptr;
     int2 *d_cij = nullptr;
-    int32_t *d_gbeg = nullptr;           // workgroup -> first chunk of its group
-    int64_t nchunks = 0, ngroups = 0;
+    int64_t nchunks = 0;
     int64_t nslots = 0;                  // physical pair slots (stored pairs + tile padding)
     int tile_R = 0;
     int soa = 0;                         // P layout: 0 pair-contiguous, 1 SoA granules of 8 pairs

@@ -896,7 +896,7 @@ dmd_scatt::~dmd_scatt()
 {
     dfree(d_e); dfree(d_edm); dfree(d_P); dfree(d_inv); dfree(d_rowptr); dfree(d_revptr); dfree(d_revpos);
     dfree(d_col); dfree(d_revcol); dfree(d_k1); dfree(d_k2); dfree(d_fwdpos); dfree(d_pk); dfree(d_cbeg);
-    dfree(d_clen); dfree(d_cij); dfree(d_gbeg); dfree(d_rhoS); dfree(d_rho1S); dfree(d_out); dfree(d_eq); dfree(d_dPH);
+    dfree(d_clen); dfree(d_cij); dfree(d_rhoS); dfree(d_rho1S); dfree(d_out); dfree(d_eq); dfree(d_dPH);
     dfree(d_in); dfree(d_in1); dfree(d_outw); dfree(d_clk);
     dfree(d_H); dfree(d_s); dfree(d_f); dfree(d_obs); dfree(d_part); dfree(d_acc_rows); dfree(d_acc_herm);
     dfree(d_y0); dfree(d_ya); dfree(d_yb); dfree(d_acc); dfree(d_w);
@@ -1186,13 +1186,6 @@ extern "C" int dmd_scatt_create(int64_t nk, int nb, int64_t n_pairs, const uint6
         int64_t f = KK(i);
         if (k1st[f] == k2nd[f]) { dpos.push_back(fwdpos[i]); dk.push_back((int32_t)k1st[f]); }
     }
-    std::vector<int32_t> gbeg;  // workgroup -> first chunk (groups of chunks of one row block)
-    const int group = lane_perm ? DMD_TILE_GROUP : DMD_TILE4_GROUP;
-    for (int64_t c = 0; c < (int64_t)cbeg.size(); c++)
-        if (gbeg.empty() || cij[c].x != cij[gbeg.back()].x || c - gbeg.back() >= group)
-            gbeg.push_back((int32_t)c);
-    gbeg.push_back((int32_t)cbeg.size());
-    h->ngroups = (int64_t)gbeg.size() - 1;
     std::vector<uint32_t> pk;
     if (R) {
         // padding slots: (0, 0) for nb <= 2 (never read), a marker for nb = 4
@@ -1218,8 +1211,7 @@ extern "C" int dmd_scatt_create(int64_t nk, int nb, int64_t n_pairs, const uint6
         (rc = dalloc_t(&h->d_acc_herm, (size_t)nk * h->nb2, "Hermitian accumulator")))
         return rc;
     if (R && ((rc = dalloc_t(&h->d_pk, nslots, "tile offsets")) || (rc = dalloc_t(&h->d_cbeg, h->nchunks, "chunks")) ||
-              (rc = dalloc_t(&h->d_clen, h->nchunks, "chunks")) || (rc = dalloc_t(&h->d_cij, h->nchunks, "chunks")) ||
-              (rc = dalloc_t(&h->d_gbeg, h->ngroups + 1, "chunk groups"))))
+              (rc = dalloc_t(&h->d_clen, h->nchunks, "chunks")) || (rc = dalloc_t(&h->d_cij, h->nchunks, "chunks"))))
         return rc;
     h->ndiag = (int64_t)dpos.size();
     if (h->ndiag) {
@@ -1253,7 +1245,6 @@ extern "C" int dmd_scatt_create(int64_t nk, int nb, int64_t n_pairs, const uint6
         DMD_HIP(hipMemcpy(h->d_cbeg, cbeg.data(), h->nchunks * 8, hipMemcpyHostToDevice));
         DMD_HIP(hipMemcpy(h->d_clen, clen.data(), h->nchunks * 4, hipMemcpyHostToDevice));
         DMD_HIP(hipMemcpy(h->d_cij, cij.data(), h->nchunks * 8, hipMemcpyHostToDevice));
-        DMD_HIP(hipMemcpy(h->d_gbeg, gbeg.data(), (h->ngroups + 1) * 4, hipMemcpyHostToDevice));
     }
     if (nslots) DMD_HIP(hipMemset(h->d_P, 0, p_words * sizeof(double2)));
     if (h->d_pscale) DMD_HIP(hipMemset(h->d_pscale, 0, (size_t)nslots * sizeof(float)));
@@ -1737,7 +1728,7 @@ int launch_raw_rows(dmd_scatt *h, const double2 *X, const double2 *Y)
 // the contraction alone: packed Hermitian rows added into d_acc_herm
 static void launch_tiles_sums(dmd_scatt *h, bool dm1)
 {
-    if (h->ngroups > 0) {
+    if (h->nchunks > 0) {
         if (h->linear)
             hipLaunchKernelGGL((k_tiles_soa<false, true>), dim3((unsigned)h->nchunks), dim3(256), 0, h->st, h->nk, h->d_P,
                                h->d_pk, h->d_cbeg, h->d_clen, h->d_cij, h->d_rhoS, h->d_rho1S, h->d_acc_herm);

@@ -99,3 +99,27 @@ def test_adjoint_of_more_components_than_one_pass():
         nine, g9 = op.adjoint_rk4(rho, 0.0, FS, 5, 1, 2, dobs, [c] * 9)
     assert np.abs(nine - one[0]).max() <= 1e-12 * abs(one[0])
     assert np.abs(g9 - g1).max() <= 1e-12 * np.abs(g1).max()
+
+
+@pytest.mark.parametrize("nk,partners", [(3, 1), (65, 20), (512, 3), (513, 9), (1100, 2), (1537, 24)])
+def test_tile_vjp_matches_the_row_kernels(nk, partners):
+    """The tile VJP, its chunks from a few pairs to several iterations of every
+    wavefront and its rows on both sides of a tile's edge, diagonal pairs included,
+    against the gather and scatter of the general path: FP64 sums in another order,
+    1e-12 of the largest element."""
+    torch = pytest.importorskip("torch")
+    torch.cuda.set_device(0)
+    rng = np.random.default_rng(nk)
+    e = random_energies(nk, 2, rng)
+    k1, k2 = random_pairs(nk, partners, rng, diag=True)
+    P1, P2 = random_P(len(k1), 2, rng)
+    rho = random_rho(nk, 2, rng)
+    v = rng.normal(size=(nk, 4)) + 1j * rng.normal(size=(nk, 4))
+    got = []
+    for kernel in (_lib.DMD_KERNEL_TILES, _lib.DMD_KERNEL_ROWS):
+        with scatt.ScatteringOperator(nk, 2, k1, k2, e) as op:
+            op.upload_P(P1, P2)
+            op.set_flags(expt=True, schrodinger=False, kernel=kernel)
+            got.append(op.vjp(31 * FS, rho, v))
+    assert np.abs(got[1]).max() > 0
+    assert np.abs(got[0] - got[1]).max() <= 1e-12 * np.abs(got[1]).max()
