@@ -38,6 +38,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 #include "dmd_internal.h"
@@ -87,11 +88,33 @@ template <typename V> __device__ __forceinline__ void cfmac_t(V &acc, V a, V b) 
     acc.y = fma(a.y, b.x, acc.y);
     acc.y = fma(-a.x, b.y, acc.y);
 }
-template <typename V> __device__ __forceinline__ V shx(V v, int m)
+// v of lane ^ M of the same 16 lanes, by data-parallel moves: no trip through the
+// LDS crossbar (M = 4 is a mirror of 8 lanes and one of 4)
+template <int CTRL> __device__ __forceinline__ int dpp(int x)
+{
+    return __builtin_amdgcn_update_dpp(0, x, CTRL, 0xF, 0xF, true);
+}
+template <int M> __device__ __forceinline__ int lane_xor(int x)
+{
+    static_assert(M == 1 || M == 2 || M == 4 || M == 8, "one lane bit of a row of 16");
+    if (M == 1) return dpp<0xB1>(x);   // quad_perm 1 0 3 2
+    if (M == 2) return dpp<0x4E>(x);   // quad_perm 2 3 0 1
+    if (M == 8) return dpp<0x128>(x);  // row_ror 8
+    return dpp<0x1B>(dpp<0x141>(x));   // row_half_mirror, then quad_perm 3 2 1 0
+}
+template <int M> __device__ __forceinline__ float lane_xor(float x)
+{
+    return __int_as_float(lane_xor<M>(__float_as_int(x)));
+}
+template <int M> __device__ __forceinline__ double lane_xor(double x)
+{
+    return __hiloint2double(lane_xor<M>(__double2hiint(x)), lane_xor<M>(__double2loint(x)));
+}
+template <int M, typename V> __device__ __forceinline__ V shx(V v)
 {
     V r;
-    r.x = __shfl_xor(v.x, m);
-    r.y = __shfl_xor(v.y, m);
+    r.x = lane_xor<M>(v.x);
+    r.y = lane_xor<M>(v.y);
     return r;
 }
 template <typename V> __device__ __forceinline__ V vadd(V a, V b)
@@ -102,18 +125,18 @@ template <typename V> __device__ __forceinline__ V vadd(V a, V b)
 }
 template <typename V> __device__ __forceinline__ V vsel(bool c, V a, V b) { return c ? a : b; }
 
-// Reduce-scatter of v[0..3] over the two lane bits m_hi, m_lo of a 4-lane
-// set: afterwards the lane with bits (h, o) holds sum over the set of v[2h+o].
-template <typename V>
-__device__ __forceinline__ V reduce4(const V v[4], int lane, int m_hi, int m_lo)
+// Reduce-scatter of v[0..3] over the two lane bits HI, LO of a 4-lane set:
+// afterwards the lane with bits (h, o) holds sum over the set of v[2h+o].
+template <int HI, int LO, typename V>
+__device__ __forceinline__ V reduce4(const V v[4], int lane)
 {
-    const bool h = (lane & m_hi) != 0, o = (lane & m_lo) != 0;
+    const bool h = (lane & HI) != 0, o = (lane & LO) != 0;
     V k0 = vsel(h, v[2], v[0]), k1 = vsel(h, v[3], v[1]);
     const V s0 = vsel(h, v[0], v[2]), s1 = vsel(h, v[1], v[3]);
-    k0 = vadd(k0, shx(s0, m_hi));
-    k1 = vadd(k1, shx(s1, m_hi));
+    k0 = vadd(k0, shx<HI>(s0));
+    k1 = vadd(k1, shx<HI>(s1));
     const V keep = vsel(o, k1, k0), send = vsel(o, k0, k1);
-    return vadd(keep, shx(send, m_lo));
+    return vadd(keep, shx<LO>(send));
 }
 
 // Loads the lane's 4 x 4 blocks of P1 and P2 of the pair record at rec,
@@ -143,6 +166,21 @@ template <typename V> struct Loader<float2, V> {
     }
 };
 template <typename V> struct Loader<bf16c, V> {
+    // a lane's part of a record as stored, and its halves converted
+    static __device__ __forceinline__ void fetch(const bf16c *rec, int l, uint4 raw[8])
+    {
+#pragma unroll
+        for (int u = 0; u < 8; u++) raw[u] = ld_stream_u4(rec + (u >> 2) * 256 + ((u & 3) * 16 + l) * 4);
+    }
+    static __device__ __forceinline__ void convert(const uint4 raw[4], V p[16])
+    {
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const uint32_t w[4] = { raw[u].x, raw[u].y, raw[u].z, raw[u].w };
+#pragma unroll
+            for (int t = 0; t < 4; t++) { p[4 * u + t].x = bf16_lo(w[t]); p[4 * u + t].y = bf16_hi(w[t]); }
+        }
+    }
     static __device__ __forceinline__ void load(const bf16c *rec, int l, V p1[16], V p2[16])
     {
 #pragma unroll
@@ -219,6 +257,15 @@ __device__ __forceinline__ void flush_block4(double *acc, int64_t base, int64_t 
 // reverse Y_k' += Lscji drho_k, increments X + X^+ (evolve_eph_linear.cpp:26-53).
 // FP32 compute: three waves per SIMD (at most 168 VGPRs); the FP64 form keeps
 // its allocation (under that bound it spills).
+// FP64 and complex64 are bound by the stream of records (8 and 4 KB per pair).
+// A BF16 record is 2 KB, so a pair's own work and the chain index -> partner row
+// -> sums -> rho_k' of the assembly weigh as much as its bytes: PRE, the BF16
+// form, has the next pair's record (32 registers as stored; P1, P2 are widened
+// where they are used), rows and indices on their way during this pair's work.
+// With the 4-lane sums by data-parallel moves: 1.59 M pairs 754 -> 619 us (4.3 ->
+// 5.25 TB/s), 59 k 57.5 -> 50, 14.5 k 25.1 -> 21.8; at two waves per SIMD 1.59 M
+// take 673.  The same order loses for complex64 (64 registers of a record ahead
+// leave two waves per SIMD: 44 k pairs 46.7 -> 58 us, 1.18 M 850 -> 856).
 template <typename PT, typename CT, bool RAW, bool YNEG, bool DM1, int R, bool LIN = false>
 __global__ __launch_bounds__(256, sizeof(CT) == 4 ? 3 : 1) void k_panels4(int64_t nk, const PT *__restrict__ P,
                                                  const float *__restrict__ pscale, const int32_t *__restrict__ k1s,
@@ -231,6 +278,7 @@ __global__ __launch_bounds__(256, sizeof(CT) == 4 ? 3 : 1) void k_panels4(int64_
 {
     using V = typename C2<CT>::T;
     constexpr int RY = DM1 ? R : 1;
+    constexpr bool PRE = std::is_same<PT, bf16c>::value && sizeof(CT) == 4 && !RAW && !DM1 && !LIN;
     __shared__ double accI[R * RS4];
     __shared__ V xI[R * 16], yI[RY * 16];
     // per 16-lane group: the pair's reverse sums G1 | G2 and the rows rho_k', 1 - rho_k'
@@ -251,14 +299,55 @@ __global__ __launch_bounds__(256, sizeof(CT) == 4 ? 3 : 1) void k_panels4(int64_
     const int a = l >> 2, b = l & 3, gi = wv * 4 + grp;
     const int64_t sb = cbeg[c];
     const int Q = clen[c] >> 2;  // the chunk length is a multiple of 4
+    // PRE: this pair's line is added at the start of the next one, before its
+    // fetches, so that only the top of the loop waits for memory
+    const int64_t s0 = sb + (int64_t)grp * Q;
+    uint4 nraw[PRE ? 8 : 1];
+    V nxv = cz<V>();
+    double2 nrv = make_double2(0, 0);
+    float nsc = 1.0f;
+    int32_t nk1 = -1, nk2 = 0, mk1 = -1, mk2 = 0;  // indices of the next pair and of the one after
+    double pv = 0.0;
+    int32_t pkp = -1;
+    auto fetch = [&](int it) {
+        if constexpr (PRE) {
+            const int64_t s = s0 + it;
+            nk1 = mk1;
+            nk2 = mk1 >= 0 ? mk2 : 0;
+            Loader<PT, V>::fetch(P + s * 512, l, nraw);
+            nxv = X[(int64_t)nk2 * 16 + l];
+            if (!LIN) nrv = rhoS[(int64_t)nk2 * 16 + l];
+            if (!LIN) nsc = pscale[s];
+            const int64_t s1 = s0 + min(it + 4, Q - 1);
+            mk1 = k1s[s1];
+            mk2 = k2s[s1];
+        }
+    };
+    if (PRE && wv < Q) {
+        mk1 = k1s[s0 + wv];
+        mk2 = k2s[s0 + wv];
+        fetch(wv);
+    }
     for (int it = wv; it < Q; it += 4) {
-        const int64_t s = sb + (int64_t)grp * Q + it;
-        const int32_t kk = k1s[s];
+        const int64_t s = s0 + it;
+        const int32_t kk = PRE ? nk1 : k1s[s];
         const bool ok = kk >= 0;
-        const int64_t kp = ok ? k2s[s] : 0;
+        const int64_t kp = PRE ? nk2 : ok ? k2s[s] : 0;
         const int lo1 = ok ? (int)(kk - I0) : 0;
         V p1[16], p2[16];
-        Loader<PT, V>::load(P + s * 512, l, p1, p2);
+        uint4 raw2[PRE ? 4 : 1];
+        const V pxv = nxv;
+        const double2 prv = nrv;
+        const float psc = nsc;
+        if constexpr (PRE) {
+            Loader<PT, V>::convert(nraw, p1);
+#pragma unroll
+            for (int u = 0; u < 4; u++) raw2[u] = nraw[4 + u];
+            if (pkp >= 0 && pv != 0.0) unsafeAtomicAdd(out + (int64_t)pkp * 16 + l, pv);
+            if (it + 4 < Q) fetch(it + 4);
+        } else {
+            Loader<PT, V>::load(P + s * 512, l, p1, p2);
+        }
         if (LIN) {
             // x slices: columns 4b.. of x (rows b of the matrices)
             V xkp[4], xk[4];
@@ -277,8 +366,8 @@ __global__ __launch_bounds__(256, sizeof(CT) == 4 ? 3 : 1) void k_panels4(int64_
                     cfma_t(f1[i], p1[4 * i + j], xkp[j]);  // X_k[4a+i]  += Lscij[4a+i][4b+j] drho_k'[4b+j]
                     cfma_t(g1[i], p2[4 * i + j], xk[j]);   // Y_k'[4a+i] += Lscji[4a+i][4b+j] drho_k[4b+j]
                 }
-            const V F1 = reduce4(f1, lane, 2, 1);  // output 4a + b
-            const V G1 = reduce4(g1, lane, 2, 1);
+            const V F1 = reduce4<2, 1>(f1, lane);  // output 4a + b
+            const V G1 = reduce4<2, 1>(g1, lane);
             if (ok) {
                 double *r1 = accI + lo1 * RS4;
                 atomicAdd(r1 + 2 * (4 * a + b), (double)F1.x);
@@ -293,7 +382,7 @@ __global__ __launch_bounds__(256, sizeof(CT) == 4 ? 3 : 1) void k_panels4(int64_
         }
         // the partner row k' staged per group; the GEMVs read x and y from LDS
         // and run one after another, so few registers beyond P stay live
-        const V xv = X[kp * 16 + l];
+        const V xv = PRE ? pxv : X[kp * 16 + l];
         __builtin_amdgcn_wave_barrier();  // the previous pair's reads of the group's rows come first
         xsc[gi][l] = xv;
         if (DM1) ysc[gi][l] = Y[kp * 16 + l];
@@ -321,7 +410,7 @@ __global__ __launch_bounds__(256, sizeof(CT) == 4 ? 3 : 1) void k_panels4(int64_
 #pragma unroll
             for (int i = 0; i < 4; i++) cfma_t(f[i], p1[4 * i + j], x);
         }
-        V F1 = reduce4(f, lane, 2, 1);  // output 4a + b
+        V F1 = reduce4<2, 1>(f, lane);  // output 4a + b
         // dm1P_k'[4b+j] += (1-rho_k)[4a+i] conj(P1[4a+i][4b+j])
 #pragma unroll
         for (int q = 0; q < 4; q++) f[q] = cz<V>();
@@ -331,8 +420,9 @@ __global__ __launch_bounds__(256, sizeof(CT) == 4 ? 3 : 1) void k_panels4(int64_
 #pragma unroll
             for (int j = 0; j < 4; j++) cfmac_t(f[j], y, p1[4 * i + j]);
         }
-        V G2 = reduce4(f, lane, 8, 4);  // output 4b + a
+        V G2 = reduce4<8, 4>(f, lane);  // output 4b + a
         // dm1P_k[4b+j] += (1-rho_k')[4a+i] P2[4a+i][4b+j]
+        if constexpr (PRE) Loader<PT, V>::convert(raw2, p2);
 #pragma unroll
         for (int q = 0; q < 4; q++) f[q] = cz<V>();
 #pragma unroll
@@ -341,7 +431,7 @@ __global__ __launch_bounds__(256, sizeof(CT) == 4 ? 3 : 1) void k_panels4(int64_
 #pragma unroll
             for (int j = 0; j < 4; j++) cfma_t(f[j], y, p2[4 * i + j]);
         }
-        V F2 = reduce4(f, lane, 8, 4);
+        V F2 = reduce4<8, 4>(f, lane);
         // Pdm_k'[4a+i] += rho_k[4b+j] conj(P2[4a+i][4b+j])
 #pragma unroll
         for (int q = 0; q < 4; q++) f[q] = cz<V>();
@@ -351,9 +441,9 @@ __global__ __launch_bounds__(256, sizeof(CT) == 4 ? 3 : 1) void k_panels4(int64_
 #pragma unroll
             for (int i = 0; i < 4; i++) cfmac_t(f[i], x, p2[4 * i + j]);
         }
-        V G1 = reduce4(f, lane, 2, 1);
+        V G1 = reduce4<2, 1>(f, lane);
         if (pscale) {  // a power of two: scaling the reduced sums is exact, 8 products instead of 32
-            const CT sc = (CT)pscale[s];
+            const CT sc = PRE ? (CT)psc : (CT)pscale[s];
             F1.x *= sc; F1.y *= sc; F2.x *= sc; F2.y *= sc;
             G1.x *= sc; G1.y *= sc; G2.x *= sc; G2.y *= sc;
         }
@@ -378,7 +468,7 @@ __global__ __launch_bounds__(256, sizeof(CT) == 4 ? 3 : 1) void k_panels4(int64_
             // upper), H' = C' + C'^+, lane (i, j) = (a, b) owns packed element l
             gsc[gi][4 * a + b] = make_double2((double)G1.x, (double)G1.y);
             gsc[gi][16 + 4 * b + a] = make_double2((double)G2.x, (double)G2.y);
-            rsc[gi][l] = rhoS[kp * 16 + l];
+            rsc[gi][l] = PRE ? prv : rhoS[kp * 16 + l];
             if (DM1) r1sc[gi][l] = rho1S[kp * 16 + l];
             __builtin_amdgcn_wave_barrier();
             const double2 *r1p = DM1 ? r1sc[gi] : nullptr;
@@ -387,9 +477,15 @@ __global__ __launch_bounds__(256, sizeof(CT) == 4 ? 3 : 1) void k_panels4(int64_
             __builtin_amdgcn_wave_barrier();
             const double v = herm_pack(cab, csc[gi][4 * b + a], a, b);  // C'_ba from lane (b, a)
             __builtin_amdgcn_wave_barrier();  // the group's LDS rows are read before the next pair writes them
-            if (rev && v != 0.0) unsafeAtomicAdd(out + kp * 16 + l, v);
+            if constexpr (PRE) {
+                pv = v;
+                pkp = rev ? (int32_t)kp : -1;
+            } else if (rev && v != 0.0) {
+                unsafeAtomicAdd(out + kp * 16 + l, v);
+            }
         }
     }
+    if (PRE && pkp >= 0 && pv != 0.0) unsafeAtomicAdd(out + (int64_t)pkp * 16 + l, pv);
     __syncthreads();
     flush_block4<RAW, DM1, R, LIN>(accI, I0, nk, rhoS, rho1S, out);
 }

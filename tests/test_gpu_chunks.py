@@ -12,7 +12,7 @@ import pytest
 sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))
 from helpers import FS, random_energies, random_P, random_rho, rel_err  # noqa: E402
 
-from denmat_dynm_development_amd import scatt  # noqa: E402
+from denmat_dynm_development_amd import _lib, scatt  # noqa: E402
 from oracle import oracle  # noqa: E402
 
 pytestmark = pytest.mark.gpu
@@ -53,6 +53,38 @@ def test_tile_pieces_match_the_oracle(torch_cuda, nb, nk, counts):
             assert rel_err(got.cpu().numpy(), ref) < 1e-12
         P1b, P2b = op.download_P()
         assert np.array_equal(P1b, P1) and np.array_equal(P2b, P2)
+
+
+@pytest.mark.parametrize("prec", [_lib.DMD_PREC_C64, _lib.DMD_PREC_BF16])
+@pytest.mark.parametrize("nk,counts", [
+    (70, [1] + [0] * 69),
+    (70, [5] + [0] * 31 + [21] + [0] * 37),  # waves with no pair, one and two
+    (40, [17] * 20 + [1] * 20),
+    (70, [64] * 70),
+    (300, [130] * 300),
+])
+def test_reduced_panels_are_exact_on_dyadic_data(torch_cuda, prec, nk, counts):
+    """P of small integers and a state of eighths: every product and partial sum of
+    the FP32 contraction is exact, so the result is the FP64 one but for the FP64
+    epilogue's roundings (1e-13 of the largest element)."""
+    torch = torch_cuda
+    nb = 4
+    rng = np.random.default_rng(nk + len(set(counts)))
+    k1, k2 = _rows(nk, counts, rng)
+    shape = (len(k1), 16, 16)
+    P1, P2 = (rng.integers(-4, 5, shape) + 1j * rng.integers(-4, 5, shape) for _ in range(2))
+    h = rng.integers(-4, 5, (nk, nb, nb)) / 16 + 1j * rng.integers(-4, 5, (nk, nb, nb)) / 16
+    rho = np.ascontiguousarray((h + h.conj().transpose(0, 2, 1)).reshape(nk, 16))
+    e = random_energies(nk, nb, rng)
+    out = []
+    for q in (_lib.DMD_PREC_FP64, prec):
+        with scatt.ScatteringOperator(nk, nb, k1, k2, e, nk_full=nk, precision=q) as op:
+            op.upload_P(P1, P2)
+            if q != _lib.DMD_PREC_FP64:
+                op.set_split(None)
+            out.append(op.eval(0.0, torch.from_numpy(rho).cuda()).cpu().numpy())
+    assert np.abs(out[0]).max() > 0
+    assert np.abs(out[1] - out[0]).max() <= 1e-13 * np.abs(out[0]).max()
 
 
 @pytest.fixture
