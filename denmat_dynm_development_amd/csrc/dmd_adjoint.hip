@@ -281,6 +281,23 @@ __device__ __forceinline__ void y_of(const double2 *r, const double2 *u, double2
             for (int m = 0; m < 2; m++) cfma(y[i * 2 + j], one_minus(r, i * 2 + m), u[m * 2 + j]);
         }
 }
+__device__ __forceinline__ void xy_of(const double2 *r, const double2 *u, double2 *x, double2 *y)
+{
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            double2 p = make_double2(0, 0), q = make_double2(0, 0);
+#pragma unroll
+            for (int m = 0; m < 2; m++) {
+                cfma(p, u[i * 2 + m], r[m * 2 + j]);
+                cfma(q, one_minus(r, i * 2 + m), u[m * 2 + j]);
+            }
+            x[i * 2 + j] = p;
+            y[i * 2 + j] = q;
+        }
+}
+
 // c -= u F1^+ (2 x 2)
 __device__ __forceinline__ void sub_u_f1(double2 *c, const double2 *u, const double2 *f1)
 {
@@ -603,7 +620,11 @@ __global__ __launch_bounds__(256) void k_adj_G(int64_t nslots, const int32_t *__
     // is a multiple of 8 workgroups, which makes the remap a bijection.
     const int64_t per = gridDim.x / 8;
     const int64_t bid = (int64_t)(blockIdx.x % 8) * per + blockIdx.x / 8;
-    const int64_t s = bid * blockDim.x + threadIdx.x;
+    // A wavefront takes 8 neighbouring lanes' slots (a granule, so whole lines of
+    // Gc) of 8 successive blocks of 64: a lane's successive slots mostly share
+    // their row k, so the wavefront reads 8 to 16 rows k instead of up to 64.
+    const int t = threadIdx.x & 63;
+    const int64_t s = (bid >> 1) * 512 + (t >> 3) * 64 + ((bid & 1) * 4 + (threadIdx.x >> 6)) * 8 + (t & 7);
     if (s >= nslots) return;
     const int32_t ka = k1[s];
     double2 *g = Gc + (s >> 3) * (8 * EP) + (s & 7);
@@ -628,10 +649,8 @@ __global__ __launch_bounds__(256) void k_adj_G(int64_t nslots, const int32_t *__
             rp[q] = rS[st * stride + bk * NB2 + q];
             up[q] = uS[st * stride + bk * NB2 + q];
         }
-        x_of(rk, uk, xk);
-        y_of(rk, uk, yk);
-        x_of(rp, up, xp);
-        y_of(rp, up, yp);
+        xy_of(rk, uk, xk, yk);
+        xy_of(rp, up, xp, yp);
 #pragma unroll
         for (int mm = 0; mm < NB2; mm++)
 #pragma unroll
@@ -945,7 +964,7 @@ extern "C" int dmd_scatt_adjoint_rk4(dmd_scatt *h, double t0, double dt, int64_t
     int pending = 0;  // stages held in rS / uS
     auto fold_G = [&]() -> int {
         if (gwords && pending > 0 && h->nslots > 0)
-            hipLaunchKernelGGL(k_adj_G, dim3((nblk(h->nslots, 256) + 7) / 8 * 8), dim3(256), 0, h->st, h->nslots,
+            hipLaunchKernelGGL(k_adj_G, dim3((2 * nblk(h->nslots, 512) + 7) / 8 * 8), dim3(256), 0, h->st, h->nslots,
                                h->d_k1, h->d_k2, pending, (int64_t)n, rS, uS, first_fold ? 1 : 0, Gc);
         if (pending > 0) first_fold = false;
         pending = 0;

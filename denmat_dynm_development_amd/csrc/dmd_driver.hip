@@ -1,7 +1,8 @@
 // dmd_driver.hip -- driver-side device code around the scattering operator:
 // the band window of evolve_driver, the coherent term, the spin-type
-// observable and the on-device fixed-step RK4 integrator (one step captured
-// in a HIP graph and replayed).
+// observable and the on-device integrators (tile and panel kernels: stages fused
+// with the assembly, launched on the stream; else an RK4 step is captured in a
+// HIP graph and replayed).
 //
 // Reference: dm_dynamics::compute (src_v4.5.7/DensityMatrix_Dynamics.h:243-278),
 // singdenmat_k::evolve_coh (src_v4.5.7/DenMat.cpp:29-55), update_dm_euler's
