@@ -622,7 +622,9 @@ __global__ __launch_bounds__(256) void k_adj_G(int64_t nslots, const int32_t *__
     const int64_t bid = (int64_t)(blockIdx.x % 8) * per + blockIdx.x / 8;
     // A wavefront takes 8 neighbouring lanes' slots (a granule, so whole lines of
     // Gc) of 8 successive blocks of 64: a lane's successive slots mostly share
-    // their row k, so the wavefront reads 8 to 16 rows k instead of up to 64.
+    // their row k, so the wavefront reads 8 to 16 rows k instead of up to 64.  The fold
+    // is bound by these gathers, 16 stages of two rows of each kind per pair:
+    // 7.76 M pairs 5.5 -> 4.3 ms, 477 k 246 -> 219 us.
     const int t = threadIdx.x & 63;
     const int64_t s = (bid >> 1) * 512 + (t >> 3) * 64 + ((bid & 1) * 4 + (threadIdx.x >> 6)) * 8 + (t & 7);
     if (s >= nslots) return;
